@@ -527,7 +527,7 @@ def measure(args, config: int, steps: int, warmup: int, with_cpu: bool) -> dict:
             "bound": "mfma", "achieved": round(result["achieved"], 1), "peak": PEAK_BF16_TFLOPS,
             "unit": "TFLOP/s", "frac": round(result["achieved"] / PEAK_BF16_TFLOPS, 4),
             "traffic": measured_traffic(config),
-            "kernel": "attn_items_kernel<256,4,*> (dense chunks: compact form, sparse chunks: pipelined form)",
+            "kernel": "attn_items_kernel<256,4> (dense chunks), attn_pair_kernel<256,4> (sparse chunks)",
             "flops_per_layer": result["flops"], "kernel_ms_per_layer": round(result["attn_ms"], 3),
             "launches_per_layer": result["launches"],
             "partials_reruns": result.get("partials_reruns", 0),

@@ -23,7 +23,6 @@ namespace {
 struct AttnArgs {
   const bf16_t* q;          // [Qc, Hq, D] chunk queries
   int64_t q_sq, q_sh;
-  int64_t q_bytes;          // extent of q in bytes (buffer range of the staged Q loads)
   const bf16_t* packed;     // [2, Lp, Hkv, D] cluster-ordered K/V
   int64_t packed_len;
   const bf16_t* korig;      // prompt-order keys from position wstart: k[pos - wstart, h, :]
@@ -141,12 +140,7 @@ struct AttnTileShape {
   static constexpr int CH = D / 8;                    // 16-byte chunks per row
   static constexpr int ROW_BYTES = D * 2;
   static constexpr int TILE_BYTES = KT * ROW_BYTES;   // one of K or V
-  // K, K, V, V tiles; the pipelined kernel adds a staging area for its
-  // epilogue (one 32-row slice per wave), the other stages in the tile buffers
-  static constexpr size_t stage_offset(bool pipe) { return pipe ? 4 * (size_t)TILE_BYTES : 0; }
-  static constexpr size_t lds_bytes(bool pipe) {
-    return 4 * (size_t)TILE_BYTES + (pipe ? (size_t)PREFILL_ROWS * ROW_BYTES : 0);
-  }
+  static constexpr size_t LDS_BYTES = 4 * (size_t)TILE_BYTES;   // K, K, V, V tiles
   static constexpr int ROWS_PER_INST = 64 / CH;       // rows one wave instruction covers
   static constexpr int INSTS = KT / ROWS_PER_INST;    // instructions per K (or V) tile
   static constexpr int PER_WAVE = INSTS / 4;
@@ -158,20 +152,14 @@ struct AttnTileShape {
 // 8 (i / 4) + 4 (l / 32) + i % 4, i < 16, which are exactly the B operand
 // P^T of the two 16-key steps of O^T (keys {0-3, 8-11 | 4-7, 12-15} and
 // {16-19, 24-27 | 20-23, 28-31}), so the probabilities never leave the lane.
-// PIPE: the next item's Q and first tiles are loaded while this item's
-// epilogue runs, which needs a staging area of its own (128 KB of LDS in all
-// at D = 256).  The kernel of the dense chunks, which run beside the index
-// build, stays at 64 KB of LDS and under 384 registers per lane so that the
-// build's kernels fit on the same compute units.
-template <int D, int G, bool PIPE>
+// This form holds one block per compute unit and stays at 64 KB of LDS and
+// under 384 registers per lane, so that the index build's kernels fit beside it
+// on the same compute units (the layer's dense chunks run beside the build).
+template <int D, int G>
 __global__ __launch_bounds__(256, 1) void attn_items_kernel(AttnArgs a) {
   using S = AttnTileShape<D>;
   constexpr int KS = D / 16;        // 16-dim steps of S^T
   constexpr int DT = D / 32;        // 32-dim tiles of O^T
-  // vector memory instructions of an item's epilogue: its rows (32 per wave,
-  // ROWS_PER_INST per store) and one LSE store
-  constexpr int EPI_STORES = 32 / S::ROWS_PER_INST + 1;
-  static_assert(EPI_STORES <= 63, "vmcnt range");
   extern __shared__ __attribute__((aligned(16))) unsigned char smem_attn[];
   __shared__ int s_items[2];
 
@@ -322,7 +310,6 @@ __global__ __launch_bounds__(256, 1) void attn_items_kernel(AttnArgs a) {
   const bf16_t* b_vp = nullptr;
   uint32_t b_rsb = 0;
   u32x4_t qr[KS];
-  bool q_staged = false;      // PIPE: the next item's Q rows are in the staging area
   auto begin = [&](const PrefillItem& r) {
     b_h = __builtin_amdgcn_readfirstlane(r.h);
     b_c = __builtin_amdgcn_readfirstlane(r.c);
@@ -353,20 +340,9 @@ __global__ __launch_bounds__(256, 1) void attn_items_kernel(AttnArgs a) {
     b_vp = uniform_ptr(vp);
     b_rsb = (uint32_t)__builtin_amdgcn_readfirstlane((int)(rs * 2));
     b_qidx = row_i >= b_qn ? -1 : (local ? b_qb + row_i : s_qslots[row_i]);
-    if (PIPE && q_staged) {
-      // the wave's rows were loaded into its staging slice during the
-      // previous item (K-tile layout): wait for its own loads, then read
-      __builtin_amdgcn_s_waitcnt(0);
-      const unsigned char* sq = smem_attn + S::stage_offset(true) + wave * 32 * S::ROW_BYTES;
+    const bf16_t* src = a.q + (int64_t)max(b_qidx, 0) * a.q_sq + (int64_t)(b_h * G + row_j) * a.q_sh + g * 8;
 #pragma unroll
-      for (int s = 0; s < KS; ++s)
-        qr[s] = *reinterpret_cast<const u32x4_t*>(sq + kbase[s & 7] + 256 * (s >> 3));
-    } else {
-      const bf16_t* src = a.q + (int64_t)max(b_qidx, 0) * a.q_sq + (int64_t)(b_h * G + row_j) * a.q_sh + g * 8;
-#pragma unroll
-      for (int s = 0; s < KS; ++s) qr[s] = *reinterpret_cast<const u32x4_t*>(src + s * 16);
-    }
-    q_staged = false;
+    for (int s = 0; s < KS; ++s) qr[s] = *reinterpret_cast<const u32x4_t*>(src + s * 16);
     issue(b_kp, b_rsb, b_nkeys, 0, kbuf_at(0), true);
     issue(b_vp, b_rsb, b_nkeys, 0, vbuf_at(0), false);
     if (b_nkeys > KT) issue(b_kp, b_rsb, b_nkeys, 1, kbuf_at(1), true);
@@ -387,8 +363,6 @@ __global__ __launch_bounds__(256, 1) void attn_items_kernel(AttnArgs a) {
     begin(rec);
   }
   int idx_n = -1;
-  bool begun_under_epilogue = false;   // PIPE: this item's first loads precede the last item's stores
-  int idx_after = -1;                  // PIPE: the item after the next one, claimed before those stores
 #ifdef SBSA_ATTN_PROBE
   int probe_k = 0;
 #endif
@@ -406,12 +380,8 @@ __global__ __launch_bounds__(256, 1) void attn_items_kernel(AttnArgs a) {
     const bool local = c < 0;
     const int ntiles = max(1, (nkeys + KT - 1) / KT);
     PROBE(idx, ntiles, qn, c);
-    if (!begun_under_epilogue) {
-      idx_n = next_index();
-      if (idx_n >= 0) rec = a.items[idx_n];
-    } else {
-      idx_n = idx_after;      // claimed, and its record loaded, before the last epilogue's stores
-    }
+    idx_n = next_index();
+    if (idx_n >= 0) rec = a.items[idx_n];
     // once, after this item's first tiles are in (every wave has read its
     // slot by then); the next item's first step publishes it
     bool prefetched = false;
@@ -556,56 +526,16 @@ __global__ __launch_bounds__(256, 1) void attn_items_kernel(AttnArgs a) {
     // code the scheduler can interleave; the general one handles the wave's
     // last active tile and the tiles past every row of the wave, whose loads
     // the wave still issues for the others.
-    // PIPE: the next item's Q rows into this wave's staging slice, in the
-    // K-tile layout (row r, 16-byte chunk c at slot (c % 16 ^ r % 16) + 16 (c / 16));
-    // issued in step 1, once the next item's query slots are published, after
-    // that step's tile loads, so the step's wait can leave them in flight
-    constexpr int QN = 32 / S::ROWS_PER_INST;      // loads per wave
-    auto stage_q = [&]() {
-      const int nh = __builtin_amdgcn_readfirstlane(rec.h), nc = __builtin_amdgcn_readfirstlane(rec.c);
-      const int nqb = __builtin_amdgcn_readfirstlane(rec.qb), nqn = __builtin_amdgcn_readfirstlane(rec.qn);
-      const uint64_t b = (uint64_t)a.q;
-      u32x4_t rsrc;
-      rsrc.x = __builtin_amdgcn_readfirstlane((uint32_t)b);
-      rsrc.y = __builtin_amdgcn_readfirstlane((uint32_t)(b >> 32)) & 0xffffu;
-      rsrc.z = (uint32_t)a.q_bytes;
-      rsrc.w = (uint32_t)BUFFER_CONFIG;
-      const uint32_t dst = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(lds_void_t*)(
-          smem_attn + S::stage_offset(true) + wave * 32 * S::ROW_BYTES));
-      const int p = lane % S::CH;
-#pragma unroll
-      for (int m = 0; m < QN; ++m) {
-        const int r = m * S::ROWS_PER_INST + lane / S::CH;
-        const int R = wave * 32 + r, i = R / G, j = R % G;
-        const int qi = i < nqn ? (nc < 0 ? nqb + i : s_qslots[i]) : -1;
-        const int cg = ((p & 15) ^ (r & 15)) + 16 * (p >> 4);
-        const uint32_t off = qi < 0 ? 0x80000000u
-                                    : (uint32_t)(((int64_t)qi * a.q_sq + (int64_t)(nh * G + j) * a.q_sh) * 2 + 16 * cg);
-        lds_dma16(rsrc, dst + m * S::ROWS_PER_INST * S::ROW_BYTES, off);
-      }
-    };
-    // returns whether this step staged the next item's Q
-    auto issue_next = [&](int t) -> bool {
+    auto issue_next = [&](int t) {
       if (t + 2 < ntiles) issue(kp, rs_bytes, nkeys, t + 2, kbuf_at(t & 1), true);
       if (t + 1 < ntiles) issue(vp, rs_bytes, nkeys, t + 1, vbuf_at((t + 1) & 1), false);
-      if (PIPE && t == 1 && idx_n >= 0 && !q_staged) {
-        stage_q();
-        q_staged = true;
-        return true;
-      }
-      return false;
     };
-    auto finish_step = [&](bool staged) {
-      if (staged) {
-        // every load but this step's QN staging loads (vmcnt QN, lgkmcnt 0)
-        __builtin_amdgcn_s_waitcnt((QN & 15) | ((QN >> 4) << 14) | (7 << 4));
-      } else {
-        __builtin_amdgcn_s_waitcnt(0);
-      }
+    auto finish_step = [&]() {
+      __builtin_amdgcn_s_waitcnt(0);
       __syncthreads();
     };
     auto step_full = [&](int t, f32x16_t& cur, f32x16_t& nxt) {
-      const bool staged = issue_next(t);
+      issue_next(t);
       mask_only(cur, t);
       u32x4_t pb[2];
       gemm_s_body(nxt, kbuf_at((t + 1) & 1));
@@ -624,12 +554,12 @@ __global__ __launch_bounds__(256, 1) void attn_items_kernel(AttnArgs a) {
         __builtin_amdgcn_sched_group_barrier(0x002, 4, 0);
       }
       gemm_pv(pb, vbuf_at(t & 1));
-      finish_step(staged);
+      finish_step();
     };
     // the general form, for the tiles around a wave's last active one; with
     // sweep set it only tracks the rows' maxima (no probabilities, no O)
     auto step = [&](int t, f32x16_t& cur, f32x16_t& nxt, bool sweep) {
-      const bool staged = issue_next(t);
+      issue_next(t);
       const bool act = t * KT <= wave_lim;
       const bool act_n = t + 1 < ntiles && (t + 1) * KT <= wave_lim;
       u32x4_t pb[2];
@@ -642,7 +572,7 @@ __global__ __launch_bounds__(256, 1) void attn_items_kernel(AttnArgs a) {
         exp_pack(cur, pb);
         gemm_pv(pb, vbuf_at(t & 1));
       }
-      finish_step(staged);
+      finish_step();
     };
 
     // Each row's probabilities are taken against a reference maximum fixed
@@ -664,13 +594,7 @@ __global__ __launch_bounds__(256, 1) void attn_items_kernel(AttnArgs a) {
         for (int e = 0; e < 16; ++e) o[dt][e] = 0.f;
       l_part = 0.f;
       lmax_all = NEG_INF;
-      if (PIPE && pass == 0 && begun_under_epilogue) {
-        // the first tiles were issued before the previous item's EPI_STORES
-        // stores: wait for every load but leave those stores in flight
-        __builtin_amdgcn_s_waitcnt((EPI_STORES & 15) | ((EPI_STORES >> 4) << 14) | (7 << 4));
-      } else {
-        __builtin_amdgcn_s_waitcnt(0);
-      }
+      __builtin_amdgcn_s_waitcnt(0);
       __syncthreads();
       prefetch_queries();
       f32x16_t sA, sB;
@@ -706,63 +630,26 @@ __global__ __launch_bounds__(256, 1) void attn_items_kernel(AttnArgs a) {
       }
     }
 
-    // PIPE: the next item's Q and first tiles load under this item's epilogue,
-    // and the item after it is claimed and its record loaded before the
-    // epilogue's stores, so that no wait of the next item waits for them
-    begun_under_epilogue = PIPE && idx_n >= 0;
-    if (PIPE && idx_n >= 0) {
-      begin(rec);
-      idx_after = next_index();
-      if (idx_after >= 0) rec = a.items[idx_after];
-    }
-
     // epilogue: normalise, then write the partial (or the local window) and
-    // its LSE.  The rows go through this wave's own 32-row slice of a staging
-    // area (PIPE: its own; otherwise the idle tile buffers), so that every
-    // store is 16 bytes per lane and whole rows per instruction: the item's
+    // its LSE.  The rows go through this wave's own 32-row slice of the idle
+    // tile buffers, so that every store is 16 bytes per lane and whole rows per instruction: the item's
     // rows are contiguous in part_o, and the G heads of a query are
     // contiguous in the window output.
     {
       const float l = halves_sum(l_part);
       const float inv = (l > 0.f) ? 1.0f / l : 0.f;
-      // PIPE: every store of the epilogue is issued by every lane (EPI_STORES
-      // per wave), through buffer resources over the item's rows: a lane
-      // without a row stores at an offset past the range, where the store is
-      // dropped.  The next item's first wait counts on that number.  The
-      // compact form keeps plain stores under the rows' conditions: the
-      // resources would take it past 384 registers per lane, and the index
-      // build's kernels would no longer fit beside its blocks.
-      if (!PIPE) {
-        if (qidx_r >= 0 && g == 0) {
-          const float lse = (l > 0.f) ? (m_ref + log2f(l)) * 0.69314718055994531f : NEG_INF;
-          float* ldst = local ? (a.local_lse ? a.local_lse + (int64_t)qidx_r * a.Hq + h * G + row_j : nullptr)
-                              : a.part_lse + (entry0 + row_i) * G + row_j;
-          if (ldst) *ldst = lse;
-        }
-      } else {
+      if (qidx_r >= 0 && g == 0) {
         const float lse = (l > 0.f) ? (m_ref + log2f(l)) * 0.69314718055994531f : NEG_INF;
-        const float* lbase;
-        int64_t lbytes, loff;
-        if (local) {
-          lbase = a.local_lse ? a.local_lse : reinterpret_cast<const float*>(a.q);
-          lbytes = a.local_lse ? (int64_t)a.Qc * a.Hq * 4 : 0;
-          loff = ((int64_t)qidx_r * a.Hq + h * G + row_j) * 4;
-        } else {
-          lbase = a.part_lse + entry0 * G;
-          lbytes = (int64_t)qn * G * 4;
-          loff = (int64_t)(row_i * G + row_j) * 4;
-        }
-        const __amdgpu_buffer_rsrc_t lrsrc = __builtin_amdgcn_make_buffer_rsrc(
-            (void*)uniform_ptr(reinterpret_cast<const bf16_t*>(lbase)), 0, (int)lbytes, BUFFER_CONFIG);
-        const int off = (qidx_r >= 0 && g == 0) ? (int)loff : OUT_OF_RANGE;
-        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(lse), lrsrc, off, 0, 0);
+        float* ldst = local ? (a.local_lse ? a.local_lse + (int64_t)qidx_r * a.Hq + h * G + row_j : nullptr)
+                            : a.part_lse + (entry0 + row_i) * G + row_j;
+        if (ldst) *ldst = lse;
       }
       // 16-byte chunk c of row r sits at chunk c ^ (r % 32) of the row.  Lane
       // (l32, g) holds dims 32 dt + 8 q4 + 4 g .. +3; a swap between the lane
       // halves (lanes l and l + 32) gives lane g = 0 all 8 dims of chunk
       // 4 dt + 2 p and lane g = 1 those of chunk 4 dt + 2 p + 1 (q4 = 2 p, 2 p + 1),
       // so each lane writes whole 16-byte chunks
-      unsigned char* stage = smem_attn + S::stage_offset(PIPE) + wave * 32 * S::ROW_BYTES;
+      unsigned char* stage = smem_attn + wave * 32 * S::ROW_BYTES;
 #pragma unroll
       for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
@@ -792,12 +679,6 @@ __global__ __launch_bounds__(256, 1) void attn_items_kernel(AttnArgs a) {
       // reads first, then the stores, so no store waits on a single read
       constexpr int NR = 32 / S::ROWS_PER_INST;
       const int c16 = lane % S::CH;
-      const bf16_t* obase = local ? a.local_o + (int64_t)qb * a.lo_sq + (int64_t)(h * G) * a.lo_sh
-                                  : a.part_o + entry0 * G * D;
-      const int64_t obytes = local ? ((int64_t)(qn - 1) * a.lo_sq + (int64_t)(G - 1) * a.lo_sh + D) * 2
-                                   : (int64_t)qn * G * D * 2;
-      __amdgpu_buffer_rsrc_t orsrc;
-      if (PIPE) orsrc = __builtin_amdgcn_make_buffer_rsrc((void*)uniform_ptr(obase), 0, (int)obytes, BUFFER_CONFIG);
 #pragma unroll
       for (int half = 0; half < 2; ++half) {
         u32x4_t rows[NR / 2];
@@ -814,25 +695,476 @@ __global__ __launch_bounds__(256, 1) void attn_items_kernel(AttnArgs a) {
           const int i = RR / G, j = RR % G;
           // read once, later, by the combine: non-temporal, kept out of the way
           // of the K/V in L2
-          if (PIPE) {
-            const int64_t roff = local ? ((int64_t)i * a.lo_sq + (int64_t)j * a.lo_sh) * 2
-                                       : (int64_t)(i * G + j) * D * 2;
-            __builtin_amdgcn_raw_buffer_store_b128(rows[mm], orsrc, i < qn ? (int)roff + 16 * c16 : OUT_OF_RANGE,
-                                                   0, 2);
-          } else {
-            bf16_t* dst = local ? a.local_o + (int64_t)(qb + i) * a.lo_sq + (int64_t)(h * G + j) * a.lo_sh
-                                : a.part_o + ((entry0 + i) * G + j) * D;
-            if (i < qn) __builtin_nontemporal_store(rows[mm], reinterpret_cast<u32x4_t*>(dst + 8 * c16));
-          }
+          bf16_t* dst = local ? a.local_o + (int64_t)(qb + i) * a.lo_sq + (int64_t)(h * G + j) * a.lo_sh
+                              : a.part_o + ((entry0 + i) * G + j) * D;
+          if (i < qn) __builtin_nontemporal_store(rows[mm], reinterpret_cast<u32x4_t*>(dst + 8 * c16));
         }
       }
     }
-    if (!PIPE && idx_n >= 0) {
+    if (idx_n >= 0) {
       __syncthreads();          // every wave is done with its staging rows
       begin(rec);
     }
   }
   PROBE(-3, 0, 0, 0);
+}
+
+
+// The form with two blocks per compute unit: 256 registers per lane and 64 KB
+// of LDS (D = 256), so a second block's matrix work covers the LDS latency, the
+// exponentials and the item boundaries of the first.  What differs from the
+// form above:
+// - no software pipeline inside a wave: S^T of tile t, its probabilities, then
+//   O^T += V^T P^T, with the loads of tile t + 1 in flight over the whole step
+//   (they are issued behind the step's one barrier and awaited at its end);
+// - the waves run the matrix parts at a raised wave priority, so that one
+//   block's exponentials and addresses fill the other's matrix time;
+// - an item's end: the next item's first tiles are issued, the first half of
+//   each row is staged (in the tile buffers those loads leave alone) and stored,
+//   the next item's Q rows are loaded into the registers that half held, and the
+//   second half follows; the first wait leaves its stores in flight;
+// - nothing that only the boundary uses lives across the tile loop (the lane
+//   number is made opaque there): a spilled register's reload would wait for
+//   every load and store in flight.
+// Bound at D = 256 by LDS: 128 KB of operand reads and 32 KB of tile writes per
+// 128 x 32 tile, 1280 cycles at 128 B/clk against 1024 of matrix work (a dense
+// chunk takes about 1300).  One MI355X, same inputs, former form -> this one: a
+// dense chunk of 8192 queries at 24576, 3564 -> 2967 us (1080 -> 1297 TFLOP/s;
+// an 8192^3 bf16 matrix product reaches 1313 there); a sparse chunk of 8192 at
+// 114688 (980K entries), 2328 -> 1846 us (750 -> 946 TFLOP/s); D = 128, a sparse
+// chunk of 3001 at 40009, 312 -> 252 us.
+template <int D, int G>
+__global__ __launch_bounds__(256, 2) void attn_pair_kernel(AttnArgs a) {
+  using S = AttnTileShape<D>;
+  constexpr int KS = D / 16;        // 16-dim steps of S^T
+  constexpr int DT = D / 32;        // 32-dim tiles of O^T
+  constexpr int SC = D / 16;        // 16-byte chunks of half a row (the epilogue stages half rows)
+  constexpr int HROWS = 64 / SC;    // half rows one store instruction covers
+  constexpr int HSTORES = 32 / HROWS;   // row stores of half an epilogue, per wave
+  static_assert(HSTORES <= 63, "vmcnt range");
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem_attn[];
+  __shared__ int s_items[2];
+  __shared__ int s_queue[16];
+  __shared__ int s_over[2];
+  __shared__ int s_qslots[PREFILL_ROWS];
+
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int l32 = lane & 31, g = lane >> 5;
+  const float NEG_INF = -INFINITY;
+  const int home = blockIdx.x & 7;
+  int probe = 0;
+
+  // per-lane addresses, as in the form above; the XORs of a step's or a tile's
+  // number are applied at the read
+  const int r0 = wave * S::ROWS_PER_INST + lane / S::CH;
+  const int cpos = lane % S::CH;
+  const uint32_t kslot0 = (uint32_t)((cpos ^ (r0 & 15)) * 16);
+  const uint32_t kslot1 = (uint32_t)((cpos ^ ((r0 + 4 * S::ROWS_PER_INST) & 15)) * 16);
+  const uint32_t vslot = (uint32_t)((cpos ^ ((r0 & 3) << 2)) * 16);
+  const uint32_t lds0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(lds_void_t*)smem_attn);
+  // K operand: row l32, chunk (2 s + g) ^ (l32 % 16) = (g ^ l32 % 16) ^ 2 s
+  const int kb = l32 * S::ROW_BYTES;
+  const int kx = 16 * (g ^ (l32 & 15));
+  // V^T operand: vbase[d] of the form above is vb + (vx ^ 64 d)
+  const int i16 = lane & 15, hh = (lane >> 4) & 1;
+  const int vb = 2 * S::TILE_BYTES + (4 * g + (i16 >> 2)) * S::ROW_BYTES + 32 * hh + 16 * ((i16 & 3) >> 1) +
+                 8 * (i16 & 1);
+  const int vx = 64 * (i16 >> 2);
+
+  if (threadIdx.x < 16) s_queue[threadIdx.x] = a.queue[threadIdx.x];
+  if (threadIdx.x < 2) s_over[threadIdx.x] = 0;
+  // Thread 0 claims work two items ahead.  The first 2 B positions of this XCD's
+  // segment (B = blocks per XCD) are paired statically, a long item with a short
+  // one; later positions come from the segment's counter, and from the other
+  // segments' once it is empty.  The counter's atomic is issued at an item's end
+  // and read after the next item's first tile, when every load has landed.
+  const int nstat = (gridDim.x % 8 == 0) ? 2 * (int)(gridDim.x / 8) : 0;
+  int pend = -1, nclaims = 0;
+  auto request = [&]() {
+    if (threadIdx.x == 0 && pend < 0 && probe < 8) pend = atomicAdd(&a.queue[16 + ((home + probe) & 7)], 1);
+  };
+  auto claim = [&]() -> int {
+    while (nclaims < 2 && nstat > 0) {
+      const int srank = (int)(blockIdx.x >> 3);
+      const int pos = nclaims++ == 0 ? srank : nstat - 1 - srank;
+      if (pos < s_queue[home]) return s_queue[8 + home] + pos;
+    }
+    for (; probe < 8; ++probe) {
+      const int x = (home + probe) & 7;
+      if (pend < 0) pend = atomicAdd(&a.queue[16 + x], 1);
+      const int pos = nstat + pend;
+      pend = -1;
+      if (pos < s_queue[x]) return s_queue[8 + x] + pos;
+    }
+    return -1;
+  };
+  // An item's record, one field per lane: field f of the record is lane f's
+  int recv = 0;
+  auto field = [&](int f) -> int { return __builtin_amdgcn_readlane(recv, f); };
+  auto load_record = [&](int idx) {
+    int ln = lane;                       // opaque: its address is not kept across the tile loop
+    asm volatile("" : "+v"(ln));
+    recv = reinterpret_cast<const int*>(a.items + max(idx, 0))[ln & 7];
+  };
+  // a cluster item's query slots straight into LDS (wave 0)
+  auto fetch_slots = [&]() {
+    if (wave != 0 || field(1) < 0) return;
+    const uint64_t b = (uint64_t)(a.qvals + field(5));
+    u32x4_t rsrc;
+    rsrc.x = __builtin_amdgcn_readfirstlane((uint32_t)b);
+    rsrc.y = __builtin_amdgcn_readfirstlane((uint32_t)(b >> 32)) & 0xffffu;
+    rsrc.z = (uint32_t)field(3) * 4u;
+    rsrc.w = (uint32_t)BUFFER_CONFIG;
+    const uint32_t dst = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(lds_void_t*)s_qslots);
+#pragma unroll
+    for (int k = 0; k < PREFILL_ROWS / G; k += 64) lds_dma4(rsrc, dst + 4 * k, (uint32_t)(lane + k) * 4u);
+  };
+
+  // the item being run
+  int i_h = 0, i_c = 0, i_qb = 0, i_qn = 0, i_nkeys = 0, i_entry0 = 0;
+  int qlim = 0;             // this lane's row: the last key it sees
+  uint64_t kp = 0, vp = 0;  // its first K and V rows
+  uint32_t rsb = 0;         // bytes from row to row
+  u32x4_t qr[KS];
+  // loads of tile t's K (or V) rows straight into LDS: the resource starts at
+  // the tile and ends with the item's last key (rows past it read as zero)
+  auto issue = [&](uint64_t base, int t, uint32_t dst, bool is_k) {
+    const uint32_t t0 = (uint32_t)(t * KT);
+    const uint64_t b = base + (uint64_t)t0 * rsb;
+    u32x4_t rs;
+    rs.x = __builtin_amdgcn_readfirstlane((uint32_t)b);
+    rs.y = __builtin_amdgcn_readfirstlane((uint32_t)(b >> 32)) & 0xffffu;
+    rs.z = ((uint32_t)i_nkeys - t0) * rsb;
+    rs.w = (uint32_t)BUFFER_CONFIG;
+    int row = r0;                        // opaque: eight offsets are not kept across the tile loop
+    asm volatile("" : "+v"(row));
+    const uint32_t off = (uint32_t)row * rsb, step = 4 * S::ROWS_PER_INST * rsb;
+#pragma unroll
+    for (int m = 0; m < S::PER_WAVE; ++m)
+      lds_dma16(rs, dst + wave * 1024 + m * 4096, off + m * step + (is_k ? (m & 1 ? kslot1 : kslot0) : vslot));
+  };
+  // the item whose record is in recv: its fields, and its first tiles' loads
+  auto begin = [&]() {
+    i_h = field(0);
+    i_c = field(1);
+    i_qb = field(2);
+    i_qn = field(3);
+    i_entry0 = field(5);
+    const bool local = i_c < 0;
+    i_nkeys = max(local ? (int)(a.chunk_start + i_qb + i_qn - a.wstart) : field(4), 0);
+    const bf16_t *k, *v;
+    if (local) {
+      k = a.korig + (int64_t)i_h * a.o_sh;
+      v = a.vorig + (int64_t)i_h * a.o_sh;
+      rsb = (uint32_t)(a.o_st * 2);
+    } else {
+      k = a.packed + ((int64_t)field(6) * a.Hkv + i_h) * D;
+      v = k + a.packed_len * a.Hkv * D;
+      rsb = (uint32_t)(a.Hkv * D * 2);
+    }
+    kp = (uint64_t)uniform_ptr(k);
+    vp = (uint64_t)uniform_ptr(v);
+    issue(kp, 0, lds0, true);
+    issue(vp, 0, lds0 + 2 * S::TILE_BYTES, false);
+  };
+  // its queries (-1 past the item's; a cluster item's slots are in LDS), their
+  // Q rows and this lane's causal limit.  Rows past the item's queries take
+  // query 0's values: they are computed like any row and never stored.
+  auto load_q = [&]() {
+    int ln = lane;                       // opaque: its addresses are not kept across the tile loop
+    asm volatile("" : "+v"(ln));
+    const int R = wave * 32 + (ln & 31);
+    const int row_i = R / G, row_j = R % G, g = ln >> 5;
+    const bool local = i_c < 0;
+    const int qidx = row_i >= i_qn ? -1 : (local ? i_qb + row_i : s_qslots[row_i]);
+    qlim = local ? (qidx < 0 ? -1 : (int)(a.chunk_start - a.wstart) + qidx) : 0x7fffffff;
+    const bf16_t* src = a.q + (int64_t)max(qidx, 0) * a.q_sq + (int64_t)(i_h * G + row_j) * a.q_sh + g * 8;
+#pragma unroll
+    for (int s = 0; s < KS; ++s) qr[s] = *reinterpret_cast<const u32x4_t*>(src + s * 16);
+  };
+
+  __syncthreads();
+  int parity = 0, over_slot = 0;
+  if (threadIdx.x == 0) {
+    s_items[0] = claim();
+    s_items[1] = s_items[0] >= 0 ? claim() : -1;
+    request();
+  }
+  __syncthreads();
+  {
+    const int idx = __builtin_amdgcn_readfirstlane(s_items[0]);
+    if (idx < 0) return;
+    load_record(idx);
+  }
+  fetch_slots();
+  __builtin_amdgcn_s_waitcnt(0);
+  __syncthreads();
+  begin();
+  load_q();
+  int idx_n = __builtin_amdgcn_readfirstlane(s_items[1]);   // the next item
+  bool after_stores = false;
+  for (;;) {
+    const bool local = i_c < 0;
+    const int ntiles = max(1, (i_nkeys + KT - 1) / KT);
+    // the last key every row of this wave sees (its first query's in the window)
+    const int first_row = wave * 32 / G;
+    const int wave_min = local && first_row < i_qn ? (int)(a.chunk_start - a.wstart) + i_qb + first_row : 0x7fffffff;
+    const int full_end = min(i_nkeys - 1, wave_min);   // tiles up to this key need no mask
+    float m_ref = 0.f, l_part = 0.f;
+    f32x16_t o[DT];
+    for (int pass = 0; pass < 3; ++pass) {
+      const bool sweep = pass == 1;
+      if (pass > 0) {
+        int z = 0;             // opaque: the rare pass's addresses are not kept
+        asm volatile("" : "+s"(z));
+        issue(kp, z, lds0, true);
+        issue(vp, z, lds0 + 2 * S::TILE_BYTES, false);
+      }
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) o[dt][e] = 0.f;
+      l_part = 0.f;
+      float lmax = NEG_INF;
+      if (after_stores)
+        __builtin_amdgcn_s_waitcnt((HSTORES & 15) | ((HSTORES >> 4) << 14) | (7 << 4));
+      else
+        __builtin_amdgcn_s_waitcnt(0);
+      after_stores = false;
+      for (int t = 0; t < ntiles; ++t) {
+        __syncthreads();
+        const uint32_t nb = ((t + 1) & 1) * S::TILE_BYTES;
+        if (t + 1 < ntiles) {
+          issue(kp, t + 1, lds0 + nb, true);
+          issue(vp, t + 1, lds0 + 2 * S::TILE_BYTES + nb, false);
+        }
+        const bool first = pass == 0 && t == 0;
+        if (first) {
+          // every wave is past the previous item's overflow flag
+          load_record(idx_n);
+          if (threadIdx.x == 0) s_over[over_slot ^ 1] = 0;
+        }
+        const int cb = (t & 1) * S::TILE_BYTES;
+        __builtin_amdgcn_s_setprio(1);
+        f32x16_t sacc;
+#pragma unroll
+        for (int e = 0; e < 16; ++e) sacc[e] = 0.f;
+        {
+          constexpr int KA = 3;
+          const int kc = kb + cb;
+          auto kread = [&](int s) -> u32x4_t {
+            return *reinterpret_cast<const u32x4_t*>(smem_attn + kc + (kx ^ (32 * (s & 7))) + 256 * (s >> 3));
+          };
+          u32x4_t ka[KA];
+#pragma unroll
+          for (int f = 0; f < KA; ++f) ka[f] = kread(f);
+#pragma unroll
+          for (int s = 0; s < KS; ++s) {
+            const u32x4_t cur = ka[s % KA];
+            if (s + KA < KS) ka[s % KA] = kread(s + KA);
+            sacc = mfma32x32x16(as_bf16x8(cur), as_bf16x8(qr[s]), sacc);
+          }
+          __builtin_amdgcn_sched_group_barrier(0x100, KA, 0);
+#pragma unroll
+          for (int f = 0; f < KS - KA; ++f) {
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+          }
+          __builtin_amdgcn_sched_group_barrier(0x008, KA, 0);
+        }
+        __builtin_amdgcn_s_setprio(0);
+        if (t * KT + KT - 1 > full_end) {
+#pragma unroll
+          for (int e = 0; e < 16; ++e) {
+            const int key = t * KT + 8 * (e >> 2) + 4 * g + (e & 3);
+            if (!(key < i_nkeys && key <= qlim)) sacc[e] = NEG_INF;
+          }
+        }
+        if (sweep || first) {
+#pragma unroll
+          for (int e = 0; e < 16; e += 4)
+            lmax = fmaxf(lmax, fmaxf(fmaxf(sacc[e], sacc[e + 1]), fmaxf(sacc[e + 2], sacc[e + 3])));
+          if (!sweep) {
+            const float mx = halves_max(lmax);
+            m_ref = (mx == NEG_INF) ? 0.f : mx * a.scale_log2;
+          }
+        }
+        if (!sweep) {
+          u32x4_t pb[2];
+          float sum = 0.f;
+#pragma unroll
+          for (int e = 0; e < 16; ++e) {
+            const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(sacc[e], a.scale_log2, -m_ref));
+            sacc[e] = p;
+            sum += p;
+          }
+          l_part += sum;
+#pragma unroll
+          for (int m = 0; m < 2; ++m) {
+            pb[m].x = pack2bf(sacc[8 * m + 0], sacc[8 * m + 1]);
+            pb[m].y = pack2bf(sacc[8 * m + 2], sacc[8 * m + 3]);
+            pb[m].z = pack2bf(sacc[8 * m + 4], sacc[8 * m + 5]);
+            pb[m].w = pack2bf(sacc[8 * m + 6], sacc[8 * m + 7]);
+          }
+          __builtin_amdgcn_s_setprio(1);
+          constexpr int NF = DT * 2;
+          constexpr int VA = 4;
+          const int vc = vb + cb;
+          u32x4_t va[VA];
+          auto vread = [&](int f) -> u32x4_t {
+            const int m = f / DT, dt = f % DT;
+            const unsigned char* p = smem_attn + vc + (vx ^ (64 * (dt & 3))) + 256 * (dt >> 2) + 16 * m * S::ROW_BYTES;
+            s16x4_t part[2];
+            part[0] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_t*)p);
+            part[1] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_t*)(p + 8 * S::ROW_BYTES));
+            u32x4_t r;
+            __builtin_memcpy(&r, part, 16);
+            return r;
+          };
+#pragma unroll
+          for (int f = 0; f < VA; ++f) va[f] = vread(f);
+#pragma unroll
+          for (int f = 0; f < NF; ++f) {
+            const u32x4_t cur = va[f % VA];
+            if (f + VA < NF) va[f % VA] = vread(f + VA);
+            o[f % DT] = mfma32x32x16(as_bf16x8(cur), as_bf16x8(pb[f / DT]), o[f % DT]);
+          }
+          __builtin_amdgcn_sched_group_barrier(0x100, 2 * VA, 0);
+#pragma unroll
+          for (int f = 0; f < NF - VA; ++f) {
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+          }
+          __builtin_amdgcn_sched_group_barrier(0x008, VA, 0);
+        }
+        __builtin_amdgcn_s_setprio(0);
+        __builtin_amdgcn_s_waitcnt(0);     // this wave's share of the next tile has landed
+        if (first && idx_n >= 0) {
+          // the next item's record is here: its query slots, and the claim of the item after it
+          fetch_slots();
+          if (threadIdx.x == 0) s_items[parity] = claim();
+          if (ntiles == 1) __builtin_amdgcn_s_waitcnt(0);
+        }
+      }
+      if (pass == 0) {
+        const float l = halves_sum(l_part);
+        const bool over = !(l <= __builtin_exp2f(OVERFLOW_LOG2));
+        if (__ballot(over) && lane == 0) s_over[over_slot] = 1;
+        __syncthreads();
+        if (!__builtin_amdgcn_readfirstlane(s_over[over_slot])) break;
+      } else if (sweep) {
+        const float mx = halves_max(lmax);
+        m_ref = (mx == NEG_INF) ? 0.f : mx * a.scale_log2;
+        __syncthreads();
+      } else {
+        __syncthreads();
+      }
+    }
+
+    // what the epilogue needs of this item, then the next item's first tiles
+    // (into K 0 and V 0: every wave is done with the tile buffers)
+    const int e_h = i_h, e_c = i_c, e_qb = i_qb, e_qn = i_qn, e_entry0 = i_entry0;
+    const bool more = idx_n >= 0;
+    over_slot ^= 1;
+    if (more) {
+      begin();
+      idx_n = __builtin_amdgcn_readfirstlane(s_items[parity]);
+      parity ^= 1;
+    }
+    {
+      int ln = lane;                     // opaque, as in load_q
+      asm volatile("" : "+v"(ln));
+      const int l32 = ln & 31, g = ln >> 5, lane = ln;
+      const int row_i = (wave * 32 + l32) / G, row_j = (wave * 32 + l32) % G;
+      const bool loc = e_c < 0;
+      const float l = halves_sum(l_part);
+      const float inv = (l > 0.f) ? 1.0f / l : 0.f;
+      {
+        const float lse = (l > 0.f) ? (m_ref + log2f(l)) * 0.69314718055994531f : NEG_INF;
+        const float* lbase;
+        int lbytes, loff;
+        if (loc) {
+          lbase = a.local_lse ? a.local_lse : reinterpret_cast<const float*>(a.q);
+          lbytes = a.local_lse ? a.Qc * a.Hq * 4 : 0;
+          loff = ((e_qb + row_i) * a.Hq + e_h * G + row_j) * 4;
+        } else {
+          lbase = a.part_lse + (int64_t)e_entry0 * G;
+          lbytes = e_qn * G * 4;
+          loff = (row_i * G + row_j) * 4;
+        }
+        const __amdgpu_buffer_rsrc_t lrsrc = __builtin_amdgcn_make_buffer_rsrc(
+            (void*)uniform_ptr(reinterpret_cast<const bf16_t*>(lbase)), 0, lbytes, BUFFER_CONFIG);
+        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(lse), lrsrc,
+                                              (row_i < e_qn && g == 0) ? loff : OUT_OF_RANGE, 0, 0);
+      }
+      // half rows through this wave's slice of K 1 and V 1: 16-byte chunk c of
+      // row r at c ^ (r % SC), whole chunks from a swap of the lane halves (as in
+      // the form above), then whole row halves per store.  Every lane issues every
+      // store, a lane without a row past the range, where it is dropped: the
+      // next item's first wait counts them.
+      unsigned char* stage = smem_attn + S::TILE_BYTES * ((wave >> 1) ? 3 : 1) + (wave & 1) * (S::TILE_BYTES / 2);
+      const bf16_t* obase = loc ? a.local_o + (int64_t)e_qb * a.lo_sq + (int64_t)(e_h * G) * a.lo_sh
+                                : a.part_o + (int64_t)e_entry0 * G * D;
+      const int64_t obytes = loc ? ((int64_t)(e_qn - 1) * a.lo_sq + (int64_t)(G - 1) * a.lo_sh + D) * 2
+                                 : (int64_t)e_qn * G * D * 2;
+      const __amdgpu_buffer_rsrc_t orsrc =
+          __builtin_amdgcn_make_buffer_rsrc((void*)uniform_ptr(obase), 0, (int)obytes, BUFFER_CONFIG);
+      const uint32_t osq = loc ? (uint32_t)(a.lo_sq * 2) : G * D * 2, osh = loc ? (uint32_t)(a.lo_sh * 2) : D * 2;
+#pragma unroll
+      for (int hf = 0; hf < 2; ++hf) {
+#pragma unroll
+        for (int dd = 0; dd < DT / 2; ++dd)
+#pragma unroll
+          for (int p = 0; p < 2; ++p) {
+            const int dt = hf * (DT / 2) + dd;
+            const int qa = 2 * p, qb2 = 2 * p + 1;
+            const uint32_t a0 = pack2bf(o[dt][4 * qa + 0] * inv, o[dt][4 * qa + 1] * inv);
+            const uint32_t a1 = pack2bf(o[dt][4 * qa + 2] * inv, o[dt][4 * qa + 3] * inv);
+            const uint32_t b0 = pack2bf(o[dt][4 * qb2 + 0] * inv, o[dt][4 * qb2 + 1] * inv);
+            const uint32_t b1 = pack2bf(o[dt][4 * qb2 + 2] * inv, o[dt][4 * qb2 + 3] * inv);
+            const auto s0 = __builtin_amdgcn_permlane32_swap(a0, b0, false, false);
+            const auto s1 = __builtin_amdgcn_permlane32_swap(a1, b1, false, false);
+            u32x4_t w;
+            w.x = s0[0];
+            w.y = s1[0];
+            w.z = s0[1];
+            w.w = s1[1];
+            const int c = (4 * dd + 2 * p + g) ^ (l32 & (SC - 1));
+            *reinterpret_cast<u32x4_t*>(stage + l32 * D + 16 * c) = w;
+          }
+        __builtin_amdgcn_wave_barrier();
+        u32x4_t rows[HSTORES];
+#pragma unroll
+        for (int m = 0; m < HSTORES; ++m) {
+          const int r = m * HROWS + lane / SC;
+          rows[m] = *reinterpret_cast<const u32x4_t*>(stage + r * D + 16 * ((lane % SC) ^ (r & (SC - 1))));
+        }
+#pragma unroll
+        for (int m = 0; m < HSTORES; ++m) {
+          const int RR = wave * 32 + m * HROWS + lane / SC;
+          const int i = RR / G, j = RR % G;
+          const uint32_t off = (uint32_t)i * osq + (uint32_t)j * osh + hf * D + 16 * (lane % SC);
+          __builtin_amdgcn_raw_buffer_store_b128(rows[m], orsrc, i < e_qn ? (int)off : OUT_OF_RANGE, 0, 2);
+        }
+        __builtin_amdgcn_wave_barrier();
+        if (hf == 0) {
+          // between the halves, when half of O's registers are free: the next item's Q rows,
+          // and the counter's atomic for the item after the next two
+          __builtin_amdgcn_sched_barrier(0);
+          asm volatile("" ::: "memory");
+          if (more) {
+            request();
+            load_q();
+          }
+          asm volatile("" ::: "memory");
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      }
+    }
+    if (!more) break;
+    after_stores = true;
+  }
 }
 
 
@@ -964,39 +1296,35 @@ __global__ __launch_bounds__(256) void combine_kernel(
   if (out_lse && (lane * E) % D == 0) out_lse[(int64_t)qi * Hq + h * G + j] = mx + logf(den);
 }
 
-template <int D, int G, bool PIPE>
-int launch_attn_kernel(const AttnArgs& a, int grid, hipStream_t stream) {
-  const size_t lds = AttnTileShape<D>::lds_bytes(PIPE);
-  static bool configured = false;
-  if (!configured) {
-    if (hipFuncSetAttribute((const void*)attn_items_kernel<D, G, PIPE>,
-                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
+// Launches one of the two forms with a grid that fills the GPU (or the caller's).
+using AttnKernel = void (*)(AttnArgs);
+template <int D>
+int launch_attn_kernel(AttnKernel kernel, int& auto_grid, const AttnArgs& a, int grid, hipStream_t stream) {
+  const size_t lds = AttnTileShape<D>::LDS_BYTES;
+  if (!auto_grid) {
+    if (hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
       return SBSA_ERR_UNSUPPORTED;
-    configured = true;
+    int dev = 0, cus = 0, occ = 0;
+    (void)hipGetDevice(&dev);
+    (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
+    (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, (const void*)kernel, 256, lds);
+    auto_grid = (cus > 0 ? cus : 256) * (occ > 0 ? occ : 1);
   }
-  static int auto_grid = 0;
-  if (grid <= 0) {
-    if (!auto_grid) {
-      int dev = 0, cus = 0, occ = 0;
-      (void)hipGetDevice(&dev);
-      (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-      (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, (const void*)attn_items_kernel<D, G, PIPE>,
-                                                         256, lds);
-      auto_grid = (cus > 0 ? cus : 256) * (occ > 0 ? occ : 1);
-    }
-    grid = auto_grid;
-  }
-  hipLaunchKernelGGL((attn_items_kernel<D, G, PIPE>), dim3(grid), dim3(256), lds, stream, a);
+  hipLaunchKernelGGL(kernel, dim3(grid > 0 ? grid : auto_grid), dim3(256), lds, stream, a);
   return SBSA_OK;
 }
 
-// the pipelined kernel for chunks with cluster items (sparse chunks, which
-// run after the index build), the compact one for dense chunks; the
-// pipelined kernel's staged Q loads address q with 31-bit offsets
+// Which form: two blocks per compute unit for chunks with cluster items; the
+// one-block form for the dense chunks, which the layer runs beside its index
+// build (the other form holds every register, and the build would wait), and for
+// windows whose rows' output offsets pass 31 bits.
 template <int D, int G>
 int launch_attn(const AttnArgs& a, int grid, hipStream_t stream) {
-  return a.packed && a.q_bytes < 0x7fffffff ? launch_attn_kernel<D, G, true>(a, grid, stream)
-                                            : launch_attn_kernel<D, G, false>(a, grid, stream);
+  static int pair_grid = 0, items_grid = 0;
+  const int64_t window_out = ((int64_t)(PREFILL_ROWS / G - 1) * a.lo_sq + (int64_t)(G - 1) * a.lo_sh + D) * 2;
+  const bool offsets_fit = window_out < INT32_MAX && (int64_t)a.Qc * a.Hq * 4 < INT32_MAX;
+  if (a.packed && offsets_fit) return launch_attn_kernel<D>(attn_pair_kernel<D, G>, pair_grid, a, grid, stream);
+  return launch_attn_kernel<D>(attn_items_kernel<D, G>, items_grid, a, grid, stream);
 }
 
 template <int D, int G>
@@ -1077,7 +1405,6 @@ int sbsa_prefill_attend(const void* q, int64_t q_sq, int64_t q_sh, int num_queri
   a.q = (const bf16_t*)q;
   a.q_sq = q_sq;
   a.q_sh = q_sh;
-  a.q_bytes = ((int64_t)(num_queries - 1) * q_sq + (int64_t)(num_q_heads - 1) * q_sh + dim) * 2;
   a.packed = (const bf16_t*)packed;
   a.packed_len = packed_len;
   a.korig = (const bf16_t*)k_orig;
