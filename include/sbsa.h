@@ -204,7 +204,8 @@ int sbsa_prefill_items(const int32_t* rev_counts, int num_kv_heads, int num_clus
  * causally.  Cluster partials: part_o [nnz, G, dim] bf16, part_lse [nnz, G];
  * the local window: local_o [Qc, Hq, dim] (strides lo_sq, lo_sh) and
  * local_lse [Qc, Hq] (null for a dense chunk, whose local_o is the output).
- * grid: persistent blocks (<= 0: as many as the device holds at once).  dim in {128, 256}, Hq/Hkv
+ * grid: persistent blocks (0: as many as the device holds at once; < 0: as many, in a form that
+ * leaves room on every compute unit for other streams' kernels).  dim in {128, 256}, Hq/Hkv
  * in {1, 2, 4, 8}. */
 int sbsa_prefill_attend(const void* q, int64_t q_sq, int64_t q_sh, int num_queries,
                         int num_q_heads, int num_kv_heads, int dim, const void* packed,

@@ -1314,16 +1314,20 @@ int launch_attn_kernel(AttnKernel kernel, int& auto_grid, const AttnArgs& a, int
   return SBSA_OK;
 }
 
-// Which form: two blocks per compute unit for chunks with cluster items; the
-// one-block form for the dense chunks, which the layer runs beside its index
-// build (the other form holds every register, and the build would wait), and for
-// windows whose rows' output offsets pass 31 bits.
+// Which form: two blocks per compute unit, unless the caller asks for room for
+// other streams' kernels (grid < 0): the one-block form then leaves registers and
+// LDS on every compute unit.  The layer asks for it for the dense chunks that run
+// beside its index build: the other form holds every register, so the build would
+// follow it (prefill of 32768: 5.5 ms with the one-block dense chunks, 6.8 with
+// these; of 131072: 42.1 and 42.7).  Alone, a dense chunk of 8192 queries at
+// 24576 takes 2967 us in the two-block form and 3458 in the other.  A window's
+// rows whose output offsets pass 31 bits go to the one-block form too.
 template <int D, int G>
 int launch_attn(const AttnArgs& a, int grid, hipStream_t stream) {
   static int pair_grid = 0, items_grid = 0;
   const int64_t window_out = ((int64_t)(PREFILL_ROWS / G - 1) * a.lo_sq + (int64_t)(G - 1) * a.lo_sh + D) * 2;
   const bool offsets_fit = window_out < INT32_MAX && (int64_t)a.Qc * a.Hq * 4 < INT32_MAX;
-  if (a.packed && offsets_fit) return launch_attn_kernel<D>(attn_pair_kernel<D, G>, pair_grid, a, grid, stream);
+  if (grid >= 0 && offsets_fit) return launch_attn_kernel<D>(attn_pair_kernel<D, G>, pair_grid, a, grid, stream);
   return launch_attn_kernel<D>(attn_items_kernel<D, G>, items_grid, a, grid, stream);
 }
 

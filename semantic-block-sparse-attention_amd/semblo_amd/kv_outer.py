@@ -353,7 +353,9 @@ def dense_causal_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *,
                            chunk_start: int = 0, out: torch.Tensor | None = None,
                            grid: int | None = None, timing=None) -> torch.Tensor:
     """Exact causal attention of q (positions chunk_start..) over k/v rows 0..chunk_end
-    in prompt order (fused_prefill.py:155-189, the dense-prefix chunks)."""
+    in prompt order (fused_prefill.py:155-189, the dense-prefix chunks).  ``grid``: the
+    launch's blocks (None fills the GPU; -1 fills it and leaves room on every compute
+    unit for kernels of other streams)."""
     qn, hq, d = q.shape
     hkv = k.shape[1]
     g = hq // hkv

@@ -303,8 +303,9 @@ class SembloAttention:
             if timing is not None:
                 n = end - start
                 timing.add_flops(4.0 * self.head_dim * self.num_heads * (n * (start + 1) + n * (n - 1) // 2))
+            # grid -1: with room for the build's kernels on every compute unit
             dense_causal_attention(q[start:end], kk, vv, sm_scale=self.scaling, chunk_start=start,
-                                   out=out[start:end], timing=timing)
+                                   out=out[start:end], grid=-1, timing=timing)
         side = self._build_stream(q.device)
         side.wait_event(inputs_ready)
         sparse = [(st, min(length, st + step)) for st in range(0, length, step) if st > cap]

@@ -55,14 +55,22 @@ def test_sparse_chunk_at_tile_edges(hkv, g, d, qn, grid):
 
 
 @pytest.mark.parametrize("hkv,g,d", [(2, 4, 256), (1, 8, 128), (1, 1, 256)])
-@pytest.mark.parametrize("start,qn,grid", [(0, 1, None), (31, 33, None), (64, 97, 8), (200, 129, None)])
-@pytest.mark.parametrize("transposed", [False, True])
-def test_dense_chunk_at_tile_edges(hkv, g, d, start, qn, grid, transposed):
-    """Also with the output's heads outside its queries (a strided output)."""
+@pytest.mark.parametrize("start,qn,grid", [(0, 1, None), (31, 33, None), (64, 97, 8), (200, 129, None),
+                                           (0, 65, -1), (200, 129, -1)])
+@pytest.mark.parametrize("transposed,tower", [(False, False), (True, False), (False, True)])
+def test_dense_chunk_at_tile_edges(hkv, g, d, start, qn, grid, transposed, tower):
+    """Both kernel forms (grid -1 asks for the one that leaves room), also with the output's
+    heads outside its queries (a strided output) and with keys that tower over the first
+    tile's (every 61st lies along the queries' common direction: the items are redone)."""
     from semblo_amd.kv_outer import dense_causal_attention
     gen = torch.Generator().manual_seed(d + g + start + qn)
-    q = torch.randn(qn, hkv * g, d, generator=gen).to(torch.bfloat16)
+    q = torch.randn(qn, hkv * g, d, generator=gen)
     k, v = (torch.randn(start + qn, hkv, d, generator=gen).to(torch.bfloat16) for _ in range(2))
+    if tower:
+        u = torch.randn(d, generator=gen)
+        q = q + 3 * u
+        k[40::61] = (3 * u).to(torch.bfloat16)
+    q = q.to(torch.bfloat16)
     out = None
     if transposed:
         out = torch.empty(hkv * g, qn, d, dtype=torch.bfloat16, device=DEV).transpose(0, 1)
