@@ -119,6 +119,38 @@ int sbsa_bucket_layout(const int32_t* assign, int64_t length, int num_clusters, 
                        int32_t* inverse, int32_t* total_out, void* workspace,
                        size_t workspace_bytes, hipStream_t stream);
 
+/* The block build of several KV heads without a host read (the same fit as
+ * sbsa_kmeans_iterate per head, the same layout as sbsa_bucket_layout).  The
+ * reference draws from one generator, head after head: a permutation of the keys,
+ * one of the sample, and one of the sample per iteration that leaves a cluster
+ * empty (flat_index.py:237-283).  Head h's draws thus depend on the restarts
+ * of the heads before it; at most `ahead` per head, so head h is fitted for every
+ * number 0 .. ahead h of them, all fits in the same launches, and the one that
+ * holds is picked on the device.
+ *
+ * sbsa_kmeans_draws (host): the draws of every fit, from a Mersenne Twister with
+ * this 32-bit seed (torch's CPU randperm draws the same numbers): per fit the
+ * sample [fit_n] (key rows), the initial rows [C] and the restart rows
+ * [ahead][C] (sample rows), then each fit's head; sbsa_kmeans_draw_ints
+ * entries in all.  length < 2^27.
+ * sbsa_kmeans_fit: keys [length, heads, dim] bf16 at strides ld_k, ld_h; draws
+ * on the device; sizes [heads, C], indptr [heads, C+1], posting
+ * [heads, posting_cap], inverse [heads, length], codebooks
+ * [heads, 2, C, dim/2]; totals [heads + 1]: the padded totals, and the first head
+ * that left clusters empty in more than `ahead` iterations (else `heads`): that
+ * head and those after it are not valid.  dim in {64, 128, 256}, rows 16-byte
+ * aligned, the workspace 256-byte aligned. */
+int64_t sbsa_kmeans_draw_ints(int64_t fit_n, int heads, int num_clusters, int ahead);
+int sbsa_kmeans_draws(uint32_t seed, int64_t length, int64_t fit_n, int heads, int num_clusters, int ahead,
+                      int32_t* out);
+size_t sbsa_kmeans_fit_workspace_bytes(int64_t length, int64_t fit_n, int heads, int num_clusters, int dim,
+                                       int ahead, int iters);
+int sbsa_kmeans_fit(const void* keys, int64_t length, int64_t ld_k, int64_t ld_h, int heads, int dim,
+                    int router_pass, const int32_t* draws, int64_t fit_n, int num_clusters, int ahead,
+                    int iters, int align, int32_t* sizes, int32_t* indptr, int32_t* posting,
+                    int64_t posting_cap, int32_t* inverse, int32_t* totals, void* codebooks,
+                    void* workspace, size_t workspace_bytes, hipStream_t stream);
+
 /* ---- S1b: packed K/V --------------------------------------------------------
  * Replaces ProductPostingIndex.pack_prompt_kv (semblo/vllm_plugin/state.py:950-997):
  * packed [2, packed_len, Hkv, dim] gathered through posting [Hkv, width];

@@ -12,6 +12,10 @@
 //   state.py:950-997               pack_prompt_kv
 #include "sbsa_common.h"
 
+#include <atomic>
+#include <thread>
+#include <vector>
+
 namespace {
 
 // ---------------------------------------------------------------- S0 -------
@@ -100,6 +104,18 @@ __global__ void key_space_kernel(const bf16_t* __restrict__ k, int64_t length, i
   }
 }
 
+// Several fits in one launch: blockIdx.y is the fit (fits of one head share its
+// key space, and differ in their draws), or, where `pick` is given, the head,
+// whose centroids are those of fit pick[y].  Strides are in elements; a zero
+// FitBatch is a single fit.
+struct FitBatch {
+  const int32_t* head = nullptr;   // [fits] the fit's head (null: head y)
+  const int32_t* pick = nullptr;   // [heads] the fit a head uses
+  int64_t x = 0, rows = 0, cent = 0, assign = 0, bits = 0, counts = 0, src = 0, flags = 0;
+  __device__ int64_t x_at() const { return (head ? head[blockIdx.y] : (int)blockIdx.y) * x; }
+  __device__ int64_t cent_at() const { return (pick ? pick[blockIdx.y] : (int)blockIdx.y) * cent; }
+};
+
 // Argmax over centroids of round_bf16(x . c) with fp32 accumulation: the bf16
 // GEMM of flat_index.py:369 returns bf16 similarities, and torch.argmax takes
 // the first of equal maxima.
@@ -109,7 +125,11 @@ __global__ void key_space_kernel(const bf16_t* __restrict__ k, int64_t length, i
 template <int D>
 __global__ __launch_bounds__(256) void kmeans_assign_kernel(
     const bf16_t* __restrict__ x, int64_t ld_x, const int32_t* __restrict__ row_index, int64_t n,
-    const bf16_t* __restrict__ cent, int num_clusters, int32_t* __restrict__ assign) {
+    const bf16_t* __restrict__ cent, int num_clusters, int32_t* __restrict__ assign, FitBatch fb) {
+  x += fb.x_at();
+  if (row_index) row_index += blockIdx.y * fb.rows;
+  cent += fb.cent_at();
+  assign += blockIdx.y * fb.assign;
   constexpr int KS = D / 32;           // k-steps of 32
   constexpr int LDR = D + 8;           // padded LDS row (bf16 elements)
   __shared__ __attribute__((aligned(16))) bf16_t sc[64 * LDR];
@@ -211,7 +231,10 @@ constexpr int KB_WORDS = KB_ROWS / 32;
 
 __global__ __launch_bounds__(256) void kmeans_members_kernel(const int32_t* __restrict__ assign,
                                                               int64_t n, int num_clusters,
-                                                              int64_t words, uint32_t* __restrict__ bits) {
+                                                              int64_t words, uint32_t* __restrict__ bits,
+                                                              FitBatch fb) {
+  assign += blockIdx.y * fb.assign;
+  bits += blockIdx.y * fb.bits;
   extern __shared__ u32x4_t tab4[];          // [C][16] words as [C][4] 16-byte pieces
   uint32_t* tab = reinterpret_cast<uint32_t*>(tab4);
   const int64_t r0 = (int64_t)blockIdx.x * KB_ROWS;
@@ -254,7 +277,12 @@ template <int NJ>  // dims 4*lane + 256*j .. +3 for j < NJ
 __global__ __launch_bounds__(256) void kmeans_update_kernel(
     const float* __restrict__ x, int64_t ld_x, const int32_t* __restrict__ row_index,
     const uint32_t* __restrict__ bits, int64_t words, int dim, float* __restrict__ sums,
-    int32_t* __restrict__ counts) {
+    int32_t* __restrict__ counts, FitBatch fb) {
+  x += fb.x_at();
+  if (row_index) row_index += blockIdx.y * fb.rows;
+  bits += blockIdx.y * fb.bits;
+  sums += blockIdx.y * fb.cent;
+  counts += blockIdx.y * fb.counts;
   __shared__ int members[KU_LIST];
   __shared__ __attribute__((aligned(16))) float red[4][256 * NJ];
   __shared__ int wsum[4];
@@ -361,7 +389,16 @@ __global__ void kmeans_centroids_kernel(int mode, const float* __restrict__ sums
                                         const int32_t* __restrict__ row_index, int num_clusters,
                                         int dim, float* __restrict__ cent_f32,
                                         bf16_t* __restrict__ cent_bf16, int32_t* flags,
-                                        int draws) {
+                                        int draws, FitBatch fb) {
+  if (sums) sums += fb.cent_at();
+  if (counts) counts += blockIdx.y * fb.counts;
+  if (src) src += blockIdx.y * fb.src;
+  if (x) x += fb.x_at();
+  if (row_index) row_index += blockIdx.y * fb.rows;
+  if (cent_f32) cent_f32 += blockIdx.y * fb.cent;
+  cent_bf16 += blockIdx.y * fb.cent;
+  if (flags) flags += blockIdx.y * fb.flags;
+  if (mode == 0 && flags && blockIdx.x == 0 && threadIdx.x == 0) flags[0] = 0;
   const int lane = threadIdx.x & 63;
   const int c = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
   const bool update = mode == 1 || mode == 3;
@@ -430,9 +467,19 @@ __global__ void kmeans_centroids_kernel(int mode, const float* __restrict__ sums
 // Stable counting sort of positions by cluster with page-aligned runs.
 constexpr int LAYOUT_CHUNK = 1024;
 
+// The layouts of several heads in one launch (blockIdx.y is the head): strides in
+// elements of the positions, the chunk counts (with the first cluster behind them),
+// the clusters' sizes (indptr has one more per head) and the posting rows.
+struct LayoutBatch {
+  int64_t positions = 0, chunks = 0, clusters = 0, posting = 0;
+};
+
 __global__ __launch_bounds__(256) void layout_hist_kernel(const int32_t* __restrict__ assign,
                                                           int64_t length, int num_clusters,
-                                                          int32_t* __restrict__ chunk_counts) {
+                                                          int32_t* __restrict__ chunk_counts,
+                                                          LayoutBatch lb) {
+  assign += blockIdx.y * lb.positions;
+  chunk_counts += blockIdx.y * lb.chunks;
   extern __shared__ int cnt[];
   for (int c = threadIdx.x; c < num_clusters; c += 256) cnt[c] = 0;
   __syncthreads();
@@ -453,7 +500,13 @@ __global__ __launch_bounds__(1024) void layout_scan_kernel(int32_t* __restrict__
                                                            int align, int32_t* __restrict__ sizes,
                                                            int32_t* __restrict__ indptr,
                                                            int32_t* __restrict__ total_out,
-                                                           int32_t* __restrict__ first_cluster) {
+                                                           int32_t* __restrict__ first_cluster,
+                                                           LayoutBatch lb) {
+  chunk_counts += blockIdx.y * lb.chunks;
+  first_cluster += blockIdx.y * lb.chunks;
+  sizes += blockIdx.y * lb.clusters;
+  indptr += blockIdx.y * (lb.clusters ? lb.clusters + 1 : 0);
+  total_out += blockIdx.y;
   __shared__ int wsum[16];
   __shared__ int s_first;
   const int c = threadIdx.x;
@@ -494,7 +547,12 @@ __global__ __launch_bounds__(256) void layout_scatter_kernel(const int32_t* __re
                                                              int64_t length, int num_clusters,
                                                              const int32_t* __restrict__ chunk_base,
                                                              int32_t* __restrict__ posting,
-                                                             int32_t* __restrict__ inverse) {
+                                                             int32_t* __restrict__ inverse,
+                                                             LayoutBatch lb) {
+  assign += blockIdx.y * lb.positions;
+  chunk_base += blockIdx.y * lb.chunks;
+  posting += blockIdx.y * lb.posting;
+  inverse += blockIdx.y * lb.positions;
   extern __shared__ int next[];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   for (int c = threadIdx.x; c < num_clusters; c += 256)
@@ -529,7 +587,12 @@ __global__ __launch_bounds__(256) void layout_scatter_kernel(const int32_t* __re
 __global__ void layout_pad_kernel(const int32_t* __restrict__ sizes,
                                   const int32_t* __restrict__ indptr, int num_clusters,
                                   const int32_t* __restrict__ first_cluster,
-                                  int32_t* __restrict__ posting, int64_t posting_cap) {
+                                  int32_t* __restrict__ posting, int64_t posting_cap,
+                                  LayoutBatch lb) {
+  sizes += blockIdx.y * lb.clusters;
+  indptr += blockIdx.y * (lb.clusters ? lb.clusters + 1 : 0);
+  first_cluster += blockIdx.y * lb.chunks;
+  posting += blockIdx.y * lb.posting;
   const int fc = *first_cluster;
   const int32_t first_pos = posting[indptr[fc]];
   if ((int)blockIdx.x < num_clusters) {
@@ -569,6 +632,25 @@ __global__ void pack_kv_kernel(const bf16_t* __restrict__ key, const bf16_t* __r
     }
     *reinterpret_cast<u32x4_t*>(packed + ((t * packed_len + r) * num_kv_heads + h) * dim + ch * 8) = v;
   }
+}
+
+// Which fit each head takes.  Head h's fits assume 0, 1, .. `ahead` h restarts
+// before it (fit h + ahead h (h - 1) / 2 + r for r); flags[fit][iters] is the
+// number of iterations of that fit that left a cluster empty.  A head with more
+// than `ahead` of them needs restarts that were not drawn: *failed is the first
+// such head (else `heads`), and it and the later heads are not valid.
+__global__ void kmeans_resolve_kernel(const int32_t* __restrict__ flags, int iters, int heads, int ahead,
+                                      int32_t* __restrict__ pick, int32_t* __restrict__ failed) {
+  if (threadIdx.x != 0) return;
+  int restarts = 0, bad = heads;
+  for (int h = 0; h < heads; ++h) {
+    const int fit = h + ahead * (h * (h - 1) / 2) + (h < bad ? restarts : 0);
+    pick[h] = fit;
+    const int empties = flags[(int64_t)fit * (iters + 1) + iters];
+    if (empties > ahead) bad = min(bad, h);
+    restarts += empties;
+  }
+  *failed = bad;
 }
 
 // Vectorised forms of the two kernels above for rows of 64..512 elements with
@@ -629,9 +711,13 @@ template <int LPR>
 __global__ __launch_bounds__(256) void key_space_vec_kernel(const bf16_t* __restrict__ k, int64_t length,
                                                             int64_t ld_k, int router_pass,
                                                             float* __restrict__ space_f32,
-                                                            bf16_t* __restrict__ space_bf16) {
+                                                            bf16_t* __restrict__ space_bf16, int64_t ld_h) {
   constexpr int RPW = 64 / LPR;
   constexpr int D = LPR * 8;
+  // blockIdx.y: the KV head (its keys at stride ld_h, its rows behind the others')
+  k += blockIdx.y * ld_h;
+  space_f32 += (int64_t)blockIdx.y * length * D;
+  space_bf16 += (int64_t)blockIdx.y * length * D;
   const int lane = threadIdx.x & 63;
   const int64_t row = ((int64_t)blockIdx.x * 4 + (threadIdx.x >> 6)) * RPW + lane / LPR;
   const int sub = lane % LPR;
@@ -668,6 +754,66 @@ __global__ __launch_bounds__(256) void key_space_vec_kernel(const bf16_t* __rest
     *reinterpret_cast<u32x4_t*>(space_bf16 + row * D + sub * 8) =
         u32x4_t{pack2bf(s[0], s[1]), pack2bf(s[2], s[3]), pack2bf(s[4], s[5]), pack2bf(s[6], s[7])};
   }
+}
+
+void launch_key_space(const void* k, int64_t length, int64_t ld_k, int heads, int64_t ld_h, int dim, int router_pass,
+                      float* space_f32, void* space_bf16, hipStream_t stream) {
+  const int lpr = dim / 8;
+  const int64_t per_block = 4 * (64 / lpr);
+  const dim3 grid((unsigned)((length + per_block - 1) / per_block), heads);
+  auto kernel = lpr == 8 ? key_space_vec_kernel<8> : lpr == 16 ? key_space_vec_kernel<16>
+                : lpr == 32 ? key_space_vec_kernel<32> : key_space_vec_kernel<64>;
+  hipLaunchKernelGGL(kernel, grid, dim3(256), 0, stream, (const bf16_t*)k, length, ld_k, router_pass, space_f32,
+                     (bf16_t*)space_bf16, ld_h);
+}
+
+// The k-means launches of one fit or of several (the grid's y), shapes checked by the callers.
+int launch_assign(const void* x_bf16, int64_t ld_x, const int32_t* row_index, int64_t n, const void* cent_bf16,
+                  int num_clusters, int dim, int32_t* assign, int fits, const FitBatch& fb, hipStream_t stream) {
+  auto kernel = dim == 64 ? kmeans_assign_kernel<64> : dim == 128 ? kmeans_assign_kernel<128>
+                : dim == 256 ? kmeans_assign_kernel<256> : nullptr;
+  if (!kernel) return SBSA_ERR_UNSUPPORTED;
+  hipLaunchKernelGGL(kernel, dim3((unsigned)((n + 127) / 128), fits), dim3(256), 0, stream, (const bf16_t*)x_bf16,
+                     ld_x, row_index, n, (const bf16_t*)cent_bf16, num_clusters, assign, fb);
+  return SBSA_OK;
+}
+
+void launch_update(const float* x, int64_t ld_x, const int32_t* row_index, int64_t n, const int32_t* assign,
+                   int num_clusters, int dim, float* sums, int32_t* counts, uint32_t* member_bits, int fits,
+                   const FitBatch& fb, hipStream_t stream) {
+  const int64_t words = (n + KB_ROWS - 1) / KB_ROWS * KB_WORDS;
+  if (words > 0)
+    hipLaunchKernelGGL(kmeans_members_kernel, dim3((unsigned)(words / KB_WORDS), fits), dim3(256),
+                       (size_t)num_clusters * KB_WORDS * sizeof(uint32_t), stream, assign, n,
+                       num_clusters, words, member_bits, fb);
+  auto kernel = dim <= 256 ? kmeans_update_kernel<1>
+                : dim <= 512 ? kmeans_update_kernel<2>
+                : dim <= 768 ? kmeans_update_kernel<3> : kmeans_update_kernel<4>;
+  hipLaunchKernelGGL(kernel, dim3(num_clusters, fits), dim3(256), 0, stream, x, ld_x, row_index,
+                     (const uint32_t*)member_bits, words, dim, sums, counts, fb);
+}
+
+void launch_layout(const int32_t* assign, int64_t length, int num_clusters, int align, int32_t* sizes,
+                   int32_t* indptr, int32_t* posting, int64_t posting_cap, int32_t* inverse, int32_t* total_out,
+                   int32_t* chunk, int heads, hipStream_t stream) {
+  const int nchunks = (int)((length + LAYOUT_CHUNK - 1) / LAYOUT_CHUNK);
+  int32_t* first = chunk + (int64_t)nchunks * num_clusters;
+  const size_t lds = (size_t)num_clusters * sizeof(int);
+  LayoutBatch lb;
+  if (heads > 1) {
+    lb.positions = length;
+    lb.chunks = (int64_t)nchunks * num_clusters + 64;
+    lb.clusters = num_clusters;
+    lb.posting = posting_cap;
+  }
+  hipLaunchKernelGGL(layout_hist_kernel, dim3(nchunks, heads), dim3(256), lds, stream, assign, length,
+                     num_clusters, chunk, lb);
+  hipLaunchKernelGGL(layout_scan_kernel, dim3(1, heads), dim3(1024), 0, stream, chunk, nchunks,
+                     num_clusters, align, sizes, indptr, total_out, first, lb);
+  hipLaunchKernelGGL(layout_scatter_kernel, dim3(nchunks, heads), dim3(256), lds, stream, assign, length,
+                     num_clusters, chunk, posting, inverse, lb);
+  hipLaunchKernelGGL(layout_pad_kernel, dim3(num_clusters + 64, heads), dim3(256), 0, stream, sizes, indptr,
+                     num_clusters, first, posting, posting_cap, lb);
 }
 
 bool vec_rows_ok(const void* p, int64_t ld, int dim) {
@@ -709,15 +855,7 @@ int sbsa_key_space(const void* k, int64_t length, int64_t ld_k, int dim, int rou
   if (!k || !space_f32 || !space_bf16 || length < 0 || dim < 1 || dim > 512) return SBSA_ERR_ARG;
   if (length == 0) return SBSA_OK;
   if (vec_rows_ok(k, ld_k, dim) && ((uintptr_t)space_f32 & 15) == 0 && ((uintptr_t)space_bf16 & 15) == 0) {
-    const int lpr = dim / 8;
-    const int64_t per_block = 4 * (64 / lpr);
-    const dim3 grid((unsigned)((length + per_block - 1) / per_block));
-    switch (lpr) {
-      case 8: hipLaunchKernelGGL(key_space_vec_kernel<8>, grid, dim3(256), 0, stream, (const bf16_t*)k, length, ld_k, router_pass, space_f32, (bf16_t*)space_bf16); break;
-      case 16: hipLaunchKernelGGL(key_space_vec_kernel<16>, grid, dim3(256), 0, stream, (const bf16_t*)k, length, ld_k, router_pass, space_f32, (bf16_t*)space_bf16); break;
-      case 32: hipLaunchKernelGGL(key_space_vec_kernel<32>, grid, dim3(256), 0, stream, (const bf16_t*)k, length, ld_k, router_pass, space_f32, (bf16_t*)space_bf16); break;
-      default: hipLaunchKernelGGL(key_space_vec_kernel<64>, grid, dim3(256), 0, stream, (const bf16_t*)k, length, ld_k, router_pass, space_f32, (bf16_t*)space_bf16); break;
-    }
+    launch_key_space(k, length, ld_k, 1, 0, dim, router_pass, space_f32, space_bf16, stream);
     SBSA_CHECK_LAUNCH();
     return SBSA_OK;
   }
@@ -734,25 +872,8 @@ int sbsa_kmeans_assign(const void* x_bf16, int64_t ld_x, const int32_t* row_inde
   if (!x_bf16 || !cent_bf16 || !assign || n < 0 || num_clusters < 1) return SBSA_ERR_ARG;
   if (ld_x % 8) return SBSA_ERR_ARG;
   if (n == 0) return SBSA_OK;
-  dim3 grid((unsigned)((n + 127) / 128));
-  switch (dim) {
-    case 64:
-      hipLaunchKernelGGL(kmeans_assign_kernel<64>, grid, dim3(256), 0, stream, (const bf16_t*)x_bf16,
-                         ld_x, row_index, n, (const bf16_t*)cent_bf16, num_clusters, assign);
-      break;
-    case 128:
-      hipLaunchKernelGGL(kmeans_assign_kernel<128>, grid, dim3(256), 0, stream,
-                         (const bf16_t*)x_bf16, ld_x, row_index, n, (const bf16_t*)cent_bf16,
-                         num_clusters, assign);
-      break;
-    case 256:
-      hipLaunchKernelGGL(kmeans_assign_kernel<256>, grid, dim3(256), 0, stream,
-                         (const bf16_t*)x_bf16, ld_x, row_index, n, (const bf16_t*)cent_bf16,
-                         num_clusters, assign);
-      break;
-    default:
-      return SBSA_ERR_UNSUPPORTED;
-  }
+  const int rc = launch_assign(x_bf16, ld_x, row_index, n, cent_bf16, num_clusters, dim, assign, 1, FitBatch{}, stream);
+  if (rc) return rc;
   SBSA_CHECK_LAUNCH();
   return SBSA_OK;
 }
@@ -773,16 +894,7 @@ int sbsa_kmeans_update(const float* x, int64_t ld_x, const int32_t* row_index, i
     return SBSA_ERR_UNSUPPORTED;
   if (member_bits_bytes < sbsa_kmeans_member_bits_bytes(n, num_clusters)) return SBSA_ERR_CAPACITY;
   if (((uintptr_t)member_bits & 15) != 0) return SBSA_ERR_ARG;
-  const int64_t words = (n + KB_ROWS - 1) / KB_ROWS * KB_WORDS;
-  if (words > 0)
-    hipLaunchKernelGGL(kmeans_members_kernel, dim3((unsigned)(words / KB_WORDS)), dim3(256),
-                       (size_t)num_clusters * KB_WORDS * sizeof(uint32_t), stream, assign, n,
-                       num_clusters, words, member_bits);
-  auto kernel = dim <= 256 ? kmeans_update_kernel<1>
-                : dim <= 512 ? kmeans_update_kernel<2>
-                : dim <= 768 ? kmeans_update_kernel<3> : kmeans_update_kernel<4>;
-  hipLaunchKernelGGL(kernel, dim3(num_clusters), dim3(256), 0, stream, x, ld_x, row_index,
-                     (const uint32_t*)member_bits, words, dim, sums, counts);
+  launch_update(x, ld_x, row_index, n, assign, num_clusters, dim, sums, counts, member_bits, 1, FitBatch{}, stream);
   SBSA_CHECK_LAUNCH();
   return SBSA_OK;
 }
@@ -798,7 +910,7 @@ int sbsa_kmeans_centroids(int mode, const float* sums, const int32_t* counts,
   if (mode == 2 && !sums) return SBSA_ERR_ARG;
   hipLaunchKernelGGL(kmeans_centroids_kernel, dim3((num_clusters + 3) / 4), dim3(256), 0, stream,
                      mode, sums, counts, src_rows, x, ld_x, row_index, num_clusters, dim, cent_f32,
-                     (bf16_t*)cent_bf16, (int32_t*)nullptr, 0);
+                     (bf16_t*)cent_bf16, (int32_t*)nullptr, 0, FitBatch{});
   SBSA_CHECK_LAUNCH();
   return SBSA_OK;
 }
@@ -827,7 +939,7 @@ int sbsa_kmeans_iterate(const void* x_bf16, const float* x_f32, int64_t ld_x,
       hipLaunchKernelGGL(kmeans_centroids_kernel, dim3((num_clusters + 3) / 4), dim3(256), 0,
                          stream, 3, sums, counts, restart_rows, x_f32, ld_x, row_index,
                          num_clusters, dim, cent_f32, (bf16_t*)cent_bf16, restart_flags + it,
-                         restart_draws);
+                         restart_draws, FitBatch{});
       SBSA_CHECK_LAUNCH();
     }
     if (rc != SBSA_OK) return rc;
@@ -850,18 +962,8 @@ int sbsa_bucket_layout(const int32_t* assign, int64_t length, int num_clusters, 
   if (workspace_bytes < sbsa_bucket_layout_workspace_bytes(length, num_clusters)) return SBSA_ERR_CAPACITY;
   int64_t bound = length + (int64_t)num_clusters * (align - 1);
   if (posting_cap < bound) return SBSA_ERR_CAPACITY;
-  int nchunks = (int)((length + LAYOUT_CHUNK - 1) / LAYOUT_CHUNK);
-  int32_t* chunk = (int32_t*)workspace;
-  int32_t* first = chunk + (int64_t)nchunks * num_clusters;
-  size_t lds = (size_t)num_clusters * sizeof(int);
-  hipLaunchKernelGGL(layout_hist_kernel, dim3(nchunks), dim3(256), lds, stream, assign, length,
-                     num_clusters, chunk);
-  hipLaunchKernelGGL(layout_scan_kernel, dim3(1), dim3(1024), 0, stream, chunk, nchunks,
-                     num_clusters, align, sizes, indptr, total_out, first);
-  hipLaunchKernelGGL(layout_scatter_kernel, dim3(nchunks), dim3(256), lds, stream, assign, length,
-                     num_clusters, chunk, posting, inverse);
-  hipLaunchKernelGGL(layout_pad_kernel, dim3(num_clusters + 64), dim3(256), 0, stream, sizes, indptr,
-                     num_clusters, first, posting, posting_cap);
+  launch_layout(assign, length, num_clusters, align, sizes, indptr, posting, posting_cap, inverse, total_out,
+                (int32_t*)workspace, 1, stream);
   SBSA_CHECK_LAUNCH();
   return SBSA_OK;
 }
@@ -883,3 +985,215 @@ int sbsa_pack_kv(const void* key, const void* value, int64_t stride_tok, int64_t
 }
 
 }  // extern "C"
+
+namespace {
+
+int num_fits(int heads, int ahead) { return heads + ahead * (heads * (heads - 1) / 2); }
+
+// The workspace of a batched fit, in 256-byte aligned pieces.
+struct FitWorkspace {
+  size_t space_f32, space_bf16, cent_f32, cent_bf16, assign_s, bits, sums, counts, flags, pick, assign_all, layout,
+      total;
+  FitWorkspace(int64_t length, int64_t fit_n, int heads, int clusters, int dim, int ahead, int iters) {
+    size_t at = 0;
+    auto take = [&](size_t bytes) {
+      const size_t here = at;
+      at += (bytes + 255) / 256 * 256;
+      return here;
+    };
+    const size_t fits = (size_t)num_fits(heads, ahead), cd = (size_t)clusters * dim;
+    const size_t chunks = (size_t)((length + LAYOUT_CHUNK - 1) / LAYOUT_CHUNK);
+    space_f32 = take((size_t)heads * length * dim * 4);
+    space_bf16 = take((size_t)heads * length * dim * 2);
+    cent_f32 = take(fits * cd * 4);
+    cent_bf16 = take(fits * cd * 2);
+    assign_s = take(fits * fit_n * 4);
+    bits = take(fits * sbsa_kmeans_member_bits_bytes(fit_n, clusters));
+    sums = take(fits * cd * 4);
+    counts = take(fits * clusters * 4);
+    flags = take(fits * (iters + 1) * 4);
+    pick = take((size_t)heads * 4);
+    assign_all = take((size_t)heads * length * 4);
+    layout = take((size_t)heads * (chunks * clusters + 64) * 4);
+    total = at;
+  }
+};
+
+bool fit_shape_ok(int64_t length, int64_t fit_n, int heads, int clusters, int dim, int ahead, int iters) {
+  return length >= 1 && fit_n >= clusters && fit_n <= length && heads >= 1 && heads <= 64 && clusters >= 1 &&
+         clusters <= 1024 && (dim == 64 || dim == 128 || dim == 256) && ahead >= 1 && ahead <= 8 && iters >= 1;
+}
+
+// The words of the 32-bit Mersenne Twister (Matsumoto and Nishimura, 1998).
+struct Mt19937 {
+  uint32_t state[624];
+  explicit Mt19937(uint32_t seed) {
+    state[0] = seed;
+    for (uint32_t i = 1; i < 624; ++i) state[i] = 1812433253u * (state[i - 1] ^ (state[i - 1] >> 30)) + i;
+  }
+  // the next 624 words into out
+  void block(uint32_t* out) {
+    auto mix = [&](int i, int next, int far) {
+      const uint32_t y = (state[i] & 0x80000000u) | (state[next] & 0x7fffffffu);
+      state[i] = state[far] ^ (y >> 1) ^ ((y & 1u) ? 0x9908b0dfu : 0u);
+    };
+    for (int i = 0; i < 227; ++i) mix(i, i + 1, i + 397);
+    for (int i = 227; i < 623; ++i) mix(i, i + 1, i - 227);
+    mix(623, 0, 396);
+    for (int i = 0; i < 624; ++i) {
+      uint32_t y = state[i];
+      y ^= y >> 11;
+      y ^= (y << 7) & 0x9d2c5680u;
+      y ^= (y << 15) & 0xefc60000u;
+      out[i] = y ^ (y >> 18);
+    }
+  }
+};
+
+// The first `want` entries of a random permutation of 0 .. n - 1 drawn by
+// Fisher-Yates from the front (entry i swaps with i + word_i mod (n - i)), which
+// takes n - 1 words.  ident holds 0 .. n - 1 and is left so.
+void permutation_prefix(const uint32_t* words, int64_t n, int64_t want, int32_t* ident, int32_t* out) {
+  const int64_t steps = want < n - 1 ? want : n - 1;
+  for (int64_t i = 0; i < steps; ++i) {
+    const int64_t j = i + words[i] % (uint32_t)(n - i);
+    const int32_t v = ident[j];
+    ident[j] = ident[i];
+    ident[i] = v;
+    out[i] = v;
+  }
+  if (want == n) out[n - 1] = ident[n - 1];
+  // an entry was moved only into a slot j >= its own, where a later step may have
+  // found it: the drawn values and the first `steps` slots are all that changed
+  for (int64_t i = 0; i < steps; ++i) {
+    ident[out[i]] = out[i];
+    ident[i] = (int32_t)i;
+  }
+}
+
+}  // namespace
+
+extern "C" int64_t sbsa_kmeans_draw_ints(int64_t fit_n, int heads, int num_clusters, int ahead) {
+  if (fit_n < 1 || heads < 1 || num_clusters < 1 || ahead < 1) return 0;
+  return (int64_t)num_fits(heads, ahead) * (fit_n + (int64_t)(1 + ahead) * num_clusters + 1);
+}
+
+extern "C" int sbsa_kmeans_draws(uint32_t seed, int64_t length, int64_t fit_n, int heads, int num_clusters, int ahead,
+                                 int32_t* out) {
+  if (!out || !fit_shape_ok(length, fit_n, heads, num_clusters, 64, ahead, 1) || length >= (1ll << 27))
+    return SBSA_ERR_ARG;
+  try {
+    // a head takes length - 1 words, fit_n - 1, and fit_n - 1 per restart
+    const int64_t head_words = (length - 1) + (fit_n - 1);
+    const int64_t most = heads * head_words + (int64_t)ahead * heads * (fit_n - 1);
+    std::vector<uint32_t> words((size_t)(most + 623) / 624 * 624 + 624);
+    Mt19937 mt(seed);
+    for (size_t i = 0; i + 624 <= words.size(); i += 624) mt.block(words.data() + i);
+    const int64_t set = fit_n + (int64_t)(1 + ahead) * num_clusters;
+    const int fits = num_fits(heads, ahead);
+    for (int h = 0, fit = 0; h < heads; ++h)
+      for (int r = 0; r <= ahead * h; ++r) out[fits * set + fit++] = h;
+    // the fits' draws are independent of each other: shared out to a few threads
+    constexpr int THREADS = 4;
+    std::vector<int32_t> ident((size_t)length * THREADS);
+    std::atomic<int> next{0};
+    auto work = [&](int thread) {
+      int32_t* id = ident.data() + (size_t)length * thread;
+      for (int64_t i = 0; i < length; ++i) id[i] = (int32_t)i;
+      for (int fit = next++; fit < fits; fit = next++) {
+        const int h = out[fits * set + fit];
+        const int r = fit - (h + ahead * (h * (h - 1) / 2));
+        const uint32_t* w = words.data() + h * head_words + r * (fit_n - 1);
+        int32_t* at = out + fit * set;
+        permutation_prefix(w, length, fit_n, id, at);
+        w += length - 1;
+        for (int k = 0; k <= ahead; ++k)      // the initial rows, then the restarts'
+          permutation_prefix(w + k * (fit_n - 1), fit_n, num_clusters, id, at + fit_n + (int64_t)k * num_clusters);
+      }
+    };
+    std::vector<std::thread> others;
+    try {
+      for (int t = 1; t < THREADS && t < fits; ++t) others.emplace_back(work, t);
+    } catch (...) {
+      // fewer threads: the others take its share
+    }
+    work(0);
+    for (auto& t : others) t.join();
+  } catch (...) {
+    return SBSA_ERR_CAPACITY;
+  }
+  return SBSA_OK;
+}
+
+extern "C" size_t sbsa_kmeans_fit_workspace_bytes(int64_t length, int64_t fit_n, int heads, int num_clusters, int dim,
+                                                  int ahead, int iters) {
+  if (!fit_shape_ok(length, fit_n, heads, num_clusters, dim, ahead, iters)) return 0;
+  return FitWorkspace(length, fit_n, heads, num_clusters, dim, ahead, iters).total;
+}
+
+extern "C" int sbsa_kmeans_fit(const void* keys, int64_t length, int64_t ld_k, int64_t ld_h, int heads, int dim,
+                               int router_pass, const int32_t* draws, int64_t fit_n, int num_clusters, int ahead,
+                               int iters, int align, int32_t* sizes, int32_t* indptr, int32_t* posting,
+                               int64_t posting_cap, int32_t* inverse, int32_t* totals, void* codebooks,
+                               void* workspace, size_t workspace_bytes, hipStream_t stream) {
+  if (!keys || !draws || !sizes || !indptr || !posting || !inverse || !totals || !codebooks || !workspace)
+    return SBSA_ERR_ARG;
+  if (!fit_shape_ok(length, fit_n, heads, num_clusters, dim, ahead, iters) || align < 1) return SBSA_ERR_UNSUPPORTED;
+  if (!vec_rows_ok(keys, ld_k, dim) || ld_h % 8 || ((uintptr_t)workspace & 255)) return SBSA_ERR_UNSUPPORTED;
+  const FitWorkspace at(length, fit_n, heads, num_clusters, dim, ahead, iters);
+  if (workspace_bytes < at.total || posting_cap < length + (int64_t)num_clusters * (align - 1)) return SBSA_ERR_CAPACITY;
+  char* w = (char*)workspace;
+  float* space_f32 = (float*)(w + at.space_f32);
+  bf16_t* space_bf16 = (bf16_t*)(w + at.space_bf16);
+  float* cent_f32 = (float*)(w + at.cent_f32);
+  bf16_t* cent_bf16 = (bf16_t*)(w + at.cent_bf16);
+  int32_t* assign_s = (int32_t*)(w + at.assign_s);
+  uint32_t* bits = (uint32_t*)(w + at.bits);
+  float* sums = (float*)(w + at.sums);
+  int32_t* counts = (int32_t*)(w + at.counts);
+  int32_t* flags = (int32_t*)(w + at.flags);
+  int32_t* pick = (int32_t*)(w + at.pick);
+  int32_t* assign_all = (int32_t*)(w + at.assign_all);
+  const int fits = num_fits(heads, ahead);
+  const int64_t set = fit_n + (int64_t)(1 + ahead) * num_clusters;
+  const int32_t *sample = draws, *init = draws + fit_n, *restarts = init + num_clusters;
+  FitBatch fb;
+  fb.head = draws + fits * set;
+  fb.x = length * dim;
+  fb.rows = fb.src = set;
+  fb.cent = (int64_t)num_clusters * dim;
+  fb.assign = fit_n;
+  fb.bits = (int64_t)(sbsa_kmeans_member_bits_bytes(fit_n, num_clusters) / 4);
+  fb.counts = num_clusters;
+  fb.flags = iters + 1;
+  const dim3 cgrid((num_clusters + 3) / 4, fits);
+  launch_key_space(keys, length, ld_k, heads, ld_h, dim, router_pass, space_f32, space_bf16, stream);
+  hipLaunchKernelGGL(kmeans_centroids_kernel, cgrid, dim3(256), 0, stream, 0, (const float*)nullptr,
+                     (const int32_t*)nullptr, init, space_f32, (int64_t)dim, sample, num_clusters, dim, cent_f32,
+                     cent_bf16, flags, 0, fb);
+  for (int it = 0; it < iters; ++it) {
+    const int rc = launch_assign(space_bf16, dim, sample, fit_n, cent_bf16, num_clusters, dim, assign_s, fits, fb, stream);
+    if (rc) return rc;
+    launch_update(space_f32, dim, sample, fit_n, assign_s, num_clusters, dim, sums, counts, bits, fits, fb, stream);
+    hipLaunchKernelGGL(kmeans_centroids_kernel, cgrid, dim3(256), 0, stream, 3, sums, counts, restarts, space_f32,
+                       (int64_t)dim, sample, num_clusters, dim, cent_f32, cent_bf16, flags + it, ahead, fb);
+  }
+  hipLaunchKernelGGL(kmeans_resolve_kernel, dim3(1), dim3(64), 0, stream, (const int32_t*)flags, iters, heads, ahead,
+                     pick, totals + heads);
+  FitBatch hb;              // per head, with the picked fits' centroids
+  hb.pick = pick;
+  hb.x = length * dim;
+  hb.cent = (int64_t)num_clusters * dim;
+  hb.assign = length;
+  const int rc = launch_assign(space_bf16, dim, nullptr, length, cent_bf16, num_clusters, dim, assign_all, heads, hb, stream);
+  if (rc) return rc;
+  launch_layout(assign_all, length, num_clusters, align, sizes, indptr, posting, posting_cap, inverse, totals,
+                (int32_t*)(w + at.layout), heads, stream);
+  hipLaunchKernelGGL(kmeans_centroids_kernel, dim3((num_clusters + 3) / 4, heads), dim3(256), 0, stream, 2, cent_f32,
+                     (const int32_t*)nullptr, (const int32_t*)nullptr, (const float*)nullptr, (int64_t)0,
+                     (const int32_t*)nullptr, num_clusters, dim, (float*)nullptr, (bf16_t*)codebooks,
+                     (int32_t*)nullptr, 0, hb);
+  SBSA_CHECK_LAUNCH();
+  return SBSA_OK;
+}
+

@@ -33,6 +33,11 @@ SIGNATURES = {
     "sbsa_kmeans_centroids": (I32, [I32, P, P, P, P, I64, P, I32, I32, P, P, P]),
     "sbsa_bucket_layout_workspace_bytes": (SZ, [I64, I32]),
     "sbsa_bucket_layout": (I32, [P, I64, I32, I32, P, P, P, I64, P, P, P, SZ, P]),
+    "sbsa_kmeans_draw_ints": (I64, [I64, I32, I32, I32]),
+    "sbsa_kmeans_draws": (I32, [ctypes.c_uint32, I64, I64, I32, I32, I32, P]),
+    "sbsa_kmeans_fit_workspace_bytes": (SZ, [I64, I64, I32, I32, I32, I32, I32]),
+    "sbsa_kmeans_fit": (I32, [P, I64, I64, I64, I32, I32, I32, P, I64, I32, I32, I32, I32, P, P, P, I64, P, P,
+                              P, P, SZ, P]),
     "sbsa_pack_kv": (I32, [P, P, I64, I64, I32, I32, P, I64, I64, P, P]),
     "sbsa_score_select": (I32, [P, I64, I64, P, P, P, I64, I64, I32, I32, I32, I32, I32, I32,
                                 F32, F32, F32, I32, I32, P, P, P, P, P, P, P]),

@@ -49,15 +49,13 @@ class _DrawBuffers:
     and the sample and initial rows go to the device from pinned memory."""
 
     def __init__(self, length: int, fit_n: int, c: int):
+        self.perm = torch.empty(length, dtype=torch.int64)
+        self.init = torch.empty(fit_n, dtype=torch.int64)
+        self.restarts = torch.empty(RESTARTS_AHEAD, fit_n, dtype=torch.int64)
         self.sub = torch.empty(fit_n, dtype=torch.int64)        # a host-side restart's draw
-        # a head's draws (sample permutation, init rows, restart rows drawn ahead), in
-        # two sets: the next head's are drawn ahead into the set the current head is not using
-        self.sets = [_HeadDraws(length, fit_n) for _ in range(2)]
         self.pinned = torch.empty(fit_n + (1 + RESTARTS_AHEAD) * c, dtype=torch.int32,
                                   pin_memory=True)
         self.uploaded = None            # event after the last upload from `pinned`
-        self.last_empties = 0           # empty k-means iterations of the last head fitted
-        self.head_empties: dict = {}    # and of each KV head in the last build of this shape
         self.counts = None              # pinned [iterations, C] cluster counts
 
     def counts_host(self, iters: int, c: int) -> torch.Tensor:
@@ -68,42 +66,7 @@ class _DrawBuffers:
         return self.counts[:iters]
 
 
-class _HeadDraws:
-    """One KV head's permutations on the host."""
-
-    def __init__(self, length: int, fit_n: int):
-        self.perm = torch.empty(length, dtype=torch.int64)
-        self.init = torch.empty(fit_n, dtype=torch.int64)
-        self.restarts = torch.empty(RESTARTS_AHEAD, fit_n, dtype=torch.int64)
-
-
 _DRAW_BUFFERS: dict = {}
-_DRAW_AHEAD = None          # the worker thread that draws the next KV head's permutations ahead
-DRAW_AHEAD = True           # False: every head's draws on the host thread, after its counts
-DRAW_AHEAD_STATS = {"used": 0, "discarded": 0}
-
-
-_DRAW_AHEAD_LAST = None     # the last draw submitted to it
-
-
-def _draw_ahead_submit(fn, *args):
-    global _DRAW_AHEAD, _DRAW_AHEAD_LAST
-    if _DRAW_AHEAD is None:
-        from concurrent.futures import ThreadPoolExecutor
-        _DRAW_AHEAD = ThreadPoolExecutor(max_workers=1, thread_name_prefix="sbsa-draws")
-    _DRAW_AHEAD_LAST = _DRAW_AHEAD.submit(fn, *args)
-    return _DRAW_AHEAD_LAST
-
-
-def _draw_ahead_settle() -> None:
-    """Wait for a draw a build left running (one that raised before taking it): the
-    next build of the same shape draws into the same host buffers."""
-    fut = _DRAW_AHEAD_LAST
-    if fut is not None and not fut.done():
-        try:
-            fut.result()
-        except Exception:
-            pass
 
 
 def _draw_buffers(length: int, fit_n: int, c: int) -> _DrawBuffers:
@@ -114,6 +77,53 @@ def _draw_buffers(length: int, fit_n: int, c: int) -> _DrawBuffers:
             _DRAW_BUFFERS.clear()
         buf = _DRAW_BUFFERS[key] = _DrawBuffers(length, fit_n, c)
     return buf
+
+
+# The batched fit runs every head's fit for every number of restarts the heads before it
+# can have made (1 + RESTARTS_AHEAD h fits for head h).  That is worth it while a k-means
+# iteration is a chain of short launches: past BATCH_WORK (fits x sample rows x centroids)
+# the fits that are not used cost more than the host's waits between the heads
+# (one MI355X, 4 KV heads of D = 256: BATCH_FIGURES).
+BATCH_FITS = 64
+BATCH_WORK = 1 << 26
+BATCH_BYTES = 8 << 30            # of the batched fit's workspace (every head's key space at once)
+
+
+def _fit_batched(pk: torch.Tensor, *, seed: int, fit_n: int, c: int, iters: int, align: int, router_pass: bool):
+    """The whole fit and layout of every KV head in one call, with one host read at the end
+    (sbsa_kmeans_fit).  Returns (sizes, indptr, posting rows, inverse, codebooks, width), or
+    None: a shape the call does not take, or a head that left clusters empty in more
+    iterations than restarts are drawn ahead for."""
+    length, hkv, dim = pk.shape
+    dev = pk.device
+    fits = hkv + RESTARTS_AHEAD * (hkv * (hkv - 1) // 2)
+    if (not 0 <= seed or fits > BATCH_FITS or fits * fit_n * c > BATCH_WORK or dim not in (64, 128, 256)
+            or pk.stride(0) % 8 or pk.stride(1) % 8 or pk.data_ptr() % 16 or length >= 1 << 27 or iters < 1):
+        return None
+    shape = (length, fit_n, hkv, c, dim, RESTARTS_AHEAD, iters)
+    ws_bytes = _lib.query("sbsa_kmeans_fit_workspace_bytes", *shape)
+    if ws_bytes == 0 or ws_bytes > BATCH_BYTES:
+        return None
+    n_draws = _lib.query("sbsa_kmeans_draw_ints", fit_n, hkv, c, RESTARTS_AHEAD)
+    host = torch.empty(n_draws, dtype=torch.int32, pin_memory=True)
+    _lib.call("sbsa_kmeans_draws", seed & 0xffffffff, length, fit_n, hkv, c, RESTARTS_AHEAD, host.data_ptr())
+    draws = host.to(dev, non_blocking=True)
+    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
+    cap = length + c * (align - 1)
+    posting = torch.empty(hkv, cap, dtype=torch.int32, device=dev)
+    inverse = torch.empty(hkv, length, dtype=torch.int32, device=dev)
+    sizes = torch.empty(hkv, c, dtype=torch.int32, device=dev)
+    indptr = torch.empty(hkv, c + 1, dtype=torch.int32, device=dev)
+    totals = torch.empty(hkv + 1, dtype=torch.int32, device=dev)
+    codebooks = torch.empty(hkv, 2, c, dim // 2, dtype=pk.dtype, device=dev)
+    _lib.call("sbsa_kmeans_fit", _lib.ptr(pk), length, pk.stride(0), pk.stride(1), hkv, dim, int(router_pass),
+              _lib.ptr(draws), fit_n, c, RESTARTS_AHEAD, iters, align, _lib.ptr(sizes), _lib.ptr(indptr),
+              _lib.ptr(posting), cap, _lib.ptr(inverse), _lib.ptr(totals), _lib.ptr(codebooks), _lib.ptr(ws),
+              ws_bytes, _lib.stream(dev))
+    *widths, valid_heads = totals.tolist()          # the one host read
+    if valid_heads < hkv:
+        return None
+    return sizes, indptr, posting, inverse, codebooks, max(widths)
 
 
 @dataclass
@@ -219,6 +229,17 @@ class ProductPostingIndex:
         if pk.dtype != torch.bfloat16:
             raise ValueError("product_keys must be bfloat16")
 
+        if fit_trace is None and not sink:
+            fitted = _fit_batched(pk, seed=int(codebook_seed or 0), fit_n=fit_n, c=c, iters=iters,
+                                  align=max(align, 1), router_pass=bool(router_pass))
+            if fitted is not None:
+                sizes, indptr, posting_full, inverse, codebooks, width = fitted
+                return cls(codebooks=codebooks, posting_positions=posting_full[:, :width].contiguous(),
+                           bucket_indptr=indptr, bucket_sizes=sizes, prompt_length=length,
+                           max_position=length - 1, flat_clusters=c, page_align=align if align > 1 else 0,
+                           _inverse_positions=inverse)
+
+        # one head after another, with the counts read on the host per head
         space_f32 = torch.empty(length, index_dim, dtype=torch.float32, device=dev)
         space_bf = torch.empty(length, index_dim, dtype=torch.bfloat16, device=dev)
         cent_f32 = torch.empty(cf, index_dim, dtype=torch.float32, device=dev)
@@ -245,44 +266,35 @@ class ProductPostingIndex:
         ws_bytes = _lib.query("sbsa_bucket_layout_workspace_bytes", length, c)
         ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
 
-        _draw_ahead_settle()
         host = _draw_buffers(n_fit, fit_n, cf)
         counts_host = host.counts_host(n_it, cf)
 
         k_ahead = RESTARTS_AHEAD
 
-        def draws(g, hd):
+        def draw():
             """fit_flat_codebook's first two draws (flat_index.py:237-262), then the
             draws of the first k_ahead restarts (flat_index.py:277-283) made ahead: the
             GPU applies the k-th at the k-th iteration that leaves a cluster empty.
-            Returns the generator's state before each restart draw, to take back the
+            Also returns the generator's state before each restart draw, to take back the
             draws no iteration needs."""
-            torch.randperm(n_fit, generator=g, out=hd.perm)
-            torch.randperm(fit_n, generator=g, out=hd.init)
+            torch.randperm(n_fit, generator=gen, out=host.perm)
+            torch.randperm(fit_n, generator=gen, out=host.init)
             before = []
             for k in range(k_ahead):
-                before.append(g.get_state())
-                torch.randperm(fit_n, generator=g, out=hd.restarts[k])
-            return before
-
-        def upload(hd, before):
-            """The draws to the device from pinned memory."""
+                before.append(gen.get_state())
+                torch.randperm(fit_n, generator=gen, out=host.restarts[k])
+            # to the device from pinned memory
             if host.uploaded is not None:
                 host.uploaded.synchronize()     # the previous upload has left `pinned`
             total = fit_n + (1 + k_ahead) * cf
-            host.pinned[:fit_n].copy_(hd.perm[:fit_n])
-            host.pinned[fit_n:fit_n + cf].copy_(hd.init[:cf])
-            host.pinned[fit_n + cf:total].view(k_ahead, cf).copy_(hd.restarts[:, :cf])
+            host.pinned[:fit_n].copy_(host.perm[:fit_n])
+            host.pinned[fit_n:fit_n + cf].copy_(host.init[:cf])
+            host.pinned[fit_n + cf:total].view(k_ahead, cf).copy_(host.restarts[:, :cf])
             both = torch.empty(total, dtype=torch.int32, device=dev)
             both.copy_(host.pinned[:total], non_blocking=True)
             host.uploaded = torch.cuda.Event()
             host.uploaded.record()
             return both[:fit_n], both[fit_n:fit_n + cf], both[fit_n + cf:], before
-
-        cur = 0                                 # the draw set of the head being fitted
-
-        def draw():
-            return upload(host.sets[cur], draws(gen, host.sets[cur]))
 
         steps: dict = {}
 
@@ -354,22 +366,6 @@ class ProductPostingIndex:
             # the final steps are enqueued now, and again if an empty iteration past
             # those restarted on the GPU is redone below
             fit_assign = finalize(h)
-            # The next head's draws follow the restart draws this head takes, which its
-            # counts decide.  While the host waits for them, a worker draws the next head's
-            # permutations into the other draw set for a guessed number of empty iterations
-            # of this head (its number in the last build of this shape, else the last
-            # head's), from where the generator then stands: before the restart draw of that
-            # number, or after all k_ahead.  They are used if the guess holds and dropped
-            # otherwise, so the sequence of draws is the reference's either way.
-            ahead = None
-            guess = host.head_empties.get(h, host.last_empties)
-            # past k_ahead empty iterations the host draws more restarts after the counts,
-            # which no draw made ahead can follow: then nothing is drawn ahead
-            if (DRAW_AHEAD and h + 1 < hkv and fit_trace is None and iters > 0 and k_ahead > 0
-                    and guess <= k_ahead):
-                g_ahead = torch.Generator()
-                g_ahead.set_state(before_restart[guess] if guess < k_ahead else gen.get_state())
-                ahead = (guess, g_ahead, _draw_ahead_submit(draws, g_ahead, host.sets[1 - cur]))
             if counted is not None:
                 counted.synchronize()
             empties = empty_iterations(0) if iters > 0 else []
@@ -378,9 +374,8 @@ class ProductPostingIndex:
             if fit_trace is not None:
                 # the sample rows each restarted iteration drew, for its empty clusters in
                 # ascending order (the GPU applied the first k_ahead of them)
-                drawn = {it: host.sets[cur].restarts[k][:int((counts_host[it] == 0).sum())].clone().long()
+                drawn = {it: host.restarts[k][:int((counts_host[it] == 0).sum())].clone().long()
                          for k, it in enumerate(empties[:k_ahead])}
-            host.last_empties = host.head_empties[h] = len(empties)
             # the GPU restarted the first k_ahead empty iterations; the next is restarted here
             it = empties[k_ahead] if len(empties) > k_ahead else -1
             while it >= 0:
@@ -419,20 +414,6 @@ class ProductPostingIndex:
                     partition=assign_all.to('cpu', copy=True).long()))
                 steps.clear()
             if h + 1 < hkv:
-                if ahead is not None:
-                    guess, g_ahead, fut = ahead
-                    before_next = fut.result()
-                    if len(empties) == guess:
-                        # the guess held (no restart drawn on the host either): the next
-                        # head's draws are the worker's, and the generator goes on from where
-                        # the worker's copy stopped
-                        gen.set_state(g_ahead.get_state())
-                        cur = 1 - cur
-                        sample_idx, init, restart_rows, before_restart = upload(host.sets[cur],
-                                                                                before_next)
-                        DRAW_AHEAD_STATS["used"] += 1
-                        continue
-                    DRAW_AHEAD_STATS["discarded"] += 1
                 sample_idx, init, restart_rows, before_restart = draw()
         width = int(totals.max().item())
         posting = posting_full[:, :width].contiguous()
