@@ -227,6 +227,26 @@ int sbsa_prefill_items(const int32_t* rev_counts, int num_kv_heads, int num_clus
                        void* items, int64_t items_cap, int64_t partials_cap, int32_t* queue,
                        hipStream_t stream);
 
+/* The plans of consecutive sparse chunks of one prompt in one call: per chunk of
+ * chunk_queries queries (the last one what is left of num_queries) the causal
+ * sizes at its first position, the selection of its queries (vectors: their
+ * routing vectors, weights uniform, no sink), the reverse index and the work list
+ * with the chunk's window -- sbsa_causal_sizes, sbsa_score_select,
+ * sbsa_reverse_index and sbsa_prefill_items, each in one set of launches for all
+ * chunks.  first_pos: the first chunk's first position.  Outputs, one chunk after
+ * another (n chunks): causal_sizes and rev_counts [n, Hkv, C], rev_indptr
+ * [n, Hkv C + 1], nnz [n], qvals [n, chunk_queries Hkv C], items [n, items_cap],
+ * queues [n, 32]; tokens [num_queries, Hkv], theta_out (or null) the same, qmask
+ * [num_queries, Hkv, C/32], qrank [num_queries, Hkv, C].  partials_cap and
+ * last_partials_cap as in sbsa_prefill_items, for the full chunks and the last. */
+int sbsa_plan_chunks(const void* vectors, int64_t v_sq, int64_t v_sh, const void* codebooks, const int32_t* posting,
+                     int64_t width, const int32_t* indptr, const int32_t* sizes, int64_t first_pos, int num_queries,
+                     int chunk_queries, int num_q_heads, int num_kv_heads, int num_clusters, int dim,
+                     float inv_temperature, float beta, float target_tokens, int iters, int queries_per_item,
+                     int32_t* causal_sizes, int32_t* tokens, float* theta_out, int32_t* qmask, int32_t* rev_counts,
+                     int32_t* rev_indptr, int64_t* nnz, int32_t* qvals, int32_t* qrank, void* items, int64_t items_cap,
+                     int64_t partials_cap, int64_t last_partials_cap, int32_t* queues, hipStream_t stream);
+
 /* Attention over the work list (kv_outer.py:482-816; dense chunks:
  * fused_prefill.py:155-189).  q [Qc, Hq, dim] (strides q_sq, q_sh); packed
  * [2, packed_len, Hkv, dim]; k_orig/v_orig the prompt-order window whose row 0

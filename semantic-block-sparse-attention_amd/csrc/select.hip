@@ -210,12 +210,23 @@ __global__ __launch_bounds__(256) void score_select_kernel(SelectArgs a, int R) 
   }
 }
 
+// Several chunks of one prompt in one launch: blockIdx.y is the chunk, whose
+// queries follow the earlier chunks' (chunk_q each, the last one what is left of
+// total_q).  Strides are in elements; zero strides and one chunk are a single call.
+struct ChunkBatch {
+  int chunk_q = 0, total_q = 0;
+  int64_t sizes = 0, limit = 0, rev = 0, qvals = 0, items = 0;
+  __device__ int queries(int q) const { return chunk_q ? min(chunk_q, total_q - (int)blockIdx.y * chunk_q) : q; }
+};
+
 // ---------------------------------------------------------------- S3c ------
 // |{keys of cluster c with position < limit}|: the run is position-sorted.
 __global__ void causal_sizes_kernel(const int32_t* __restrict__ posting, int64_t width,
                                     const int32_t* __restrict__ indptr,
                                     const int32_t* __restrict__ sizes, int hkv, int C,
-                                    int64_t limit, int32_t* __restrict__ out) {
+                                    int64_t limit, int32_t* __restrict__ out, ChunkBatch cb) {
+  limit += blockIdx.y * cb.limit;
+  out += blockIdx.y * cb.sizes;
   int e = blockIdx.x * blockDim.x + threadIdx.x;
   if (e >= hkv * C) return;
   int h = e / C, c = e % C;
@@ -239,9 +250,16 @@ __global__ __launch_bounds__(256) void rev_pass_kernel(int pass, const int32_t* 
                                                        int32_t* __restrict__ rev_counts,
                                                        const int32_t* __restrict__ rev_indptr,
                                                        int32_t* __restrict__ qvals,
-                                                       int32_t* __restrict__ qrank) {
+                                                       int32_t* __restrict__ qrank, ChunkBatch cb) {
   __shared__ int wcnt[4];
   const int hc = blockIdx.x;
+  Q = cb.queries(Q);
+  qmask += (int64_t)blockIdx.y * cb.chunk_q * hkv * (C / 32);
+  nvis += blockIdx.y * cb.sizes;
+  rev_counts += blockIdx.y * cb.sizes;
+  rev_indptr += blockIdx.y * cb.rev;
+  qvals += blockIdx.y * cb.qvals;
+  qrank += (int64_t)blockIdx.y * cb.chunk_q * hkv * C;
   const int h = hc / C, c = hc % C;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int W = C / 32;
@@ -272,7 +290,10 @@ __global__ __launch_bounds__(256) void rev_pass_kernel(int pass, const int32_t* 
 // Exclusive scan of the Hkv*C counts (one block), total into rev_indptr[n].
 __global__ __launch_bounds__(1024) void rev_scan_kernel(const int32_t* __restrict__ counts, int n,
                                                         int32_t* __restrict__ indptr,
-                                                        int64_t* __restrict__ nnz) {
+                                                        int64_t* __restrict__ nnz, ChunkBatch cb) {
+  counts += blockIdx.y * cb.sizes;
+  indptr += blockIdx.y * cb.rev;
+  nnz += blockIdx.y;
   __shared__ int wsum[16];
   __shared__ int carry;
   if (threadIdx.x == 0) carry = 0;
@@ -347,6 +368,7 @@ __device__ __forceinline__ ItemSource item_source(const int32_t* rev_counts, con
 // queue[QUEUE_OVERFLOW]: 1 when the chunk's partial entries pass the partial
 // buffer's capacity (the list is then empty)
 constexpr int QUEUE_OVERFLOW = 24;
+constexpr int QUEUE_INTS = 32;
 
 __global__ __launch_bounds__(1024) void build_items_kernel(const int32_t* __restrict__ rev_counts,
                                                            int hkv, int C, int Qc, int QT,
@@ -355,7 +377,15 @@ __global__ __launch_bounds__(1024) void build_items_kernel(const int32_t* __rest
                                                            const int32_t* __restrict__ rev_indptr,
                                                            PrefillItem* __restrict__ items,
                                                            int32_t* __restrict__ queue,
-                                                           int64_t cap, int64_t partials_cap) {
+                                                           int64_t cap, int64_t partials_cap,
+                                                           int64_t last_partials_cap, ChunkBatch cb) {
+  Qc = cb.queries(Qc);
+  rev_counts += blockIdx.y * cb.sizes;
+  nvis += blockIdx.y * cb.sizes;
+  rev_indptr += blockIdx.y * cb.rev;
+  items += blockIdx.y * cb.items;
+  queue += blockIdx.y * QUEUE_INTS;
+  if (blockIdx.y == gridDim.y - 1) partials_cap = last_partials_cap;
   extern __shared__ int s_first[];     // [nsrc] first item of each source, then
                                        // [hkv C] sort keys and [hkv C] source order
   __shared__ int cnt[8];
@@ -469,6 +499,37 @@ __global__ __launch_bounds__(1024) void build_items_kernel(const int32_t* __rest
 }
 
 
+void launch_reverse_index(const int32_t* qmask, int num_queries, int hkv, int C, const int32_t* nvis,
+                          int32_t* rev_counts, int32_t* rev_indptr, int64_t* nnz, int32_t* qvals, int32_t* qrank,
+                          int chunks, const ChunkBatch& cb, hipStream_t stream) {
+  const int n = hkv * C;
+  hipLaunchKernelGGL(rev_pass_kernel, dim3(n, chunks), dim3(256), 0, stream, 0, qmask, num_queries, hkv, C, nvis,
+                     rev_counts, rev_indptr, qvals, qrank, cb);
+  hipLaunchKernelGGL(rev_scan_kernel, dim3(1, chunks), dim3(1024), 0, stream, rev_counts, n, rev_indptr, nnz, cb);
+  hipLaunchKernelGGL(rev_pass_kernel, dim3(n, chunks), dim3(256), 0, stream, 1, qmask, num_queries, hkv, C, nvis,
+                     rev_counts, rev_indptr, qvals, qrank, cb);
+}
+
+int launch_items(const int32_t* rev_counts, int hkv, int C, int num_queries, int queries_per_item, int has_local,
+                 const int32_t* indptr, const int32_t* nvis, const int32_t* rev_indptr, void* items,
+                 int64_t items_cap, int64_t partials_cap, int64_t last_partials_cap, int32_t* queue, int chunks,
+                 const ChunkBatch& cb, hipStream_t stream) {
+  const int nloc = has_local ? (num_queries + queries_per_item - 1) / queries_per_item : 0;
+  const size_t lds = (size_t)(nloc * hkv + 3 * hkv * C) * 4;
+  if (lds > 150 * 1024) return SBSA_ERR_UNSUPPORTED;
+  static size_t configured = 0;
+  if (lds > configured) {
+    if (hipFuncSetAttribute((const void*)build_items_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
+                            (int)lds) != hipSuccess)
+      return SBSA_ERR_UNSUPPORTED;
+    configured = lds;
+  }
+  hipLaunchKernelGGL(build_items_kernel, dim3(1, chunks), dim3(1024), lds, stream, rev_counts, hkv, C, num_queries,
+                     queries_per_item, has_local, indptr, nvis, rev_indptr, (PrefillItem*)items, queue, items_cap,
+                     partials_cap, last_partials_cap, cb);
+  return SBSA_OK;
+}
+
 }  // namespace
 
 // One instantiation per bound on the clusters a lane holds (C <= 64 NK).
@@ -561,7 +622,7 @@ int sbsa_causal_sizes(const int32_t* posting, int64_t width, const int32_t* indp
   if (!posting || !indptr || !sizes || !out || num_kv_heads < 1 || num_clusters < 1) return SBSA_ERR_ARG;
   int n = num_kv_heads * num_clusters;
   hipLaunchKernelGGL(causal_sizes_kernel, dim3((n + 255) / 256), dim3(256), 0, stream, posting,
-                     width, indptr, sizes, num_kv_heads, num_clusters, pos_limit, out);
+                     width, indptr, sizes, num_kv_heads, num_clusters, pos_limit, out, ChunkBatch{});
   SBSA_CHECK_LAUNCH();
   return SBSA_OK;
 }
@@ -574,12 +635,8 @@ int sbsa_reverse_index(const int32_t* qmask, int num_queries, int num_kv_heads, 
   if (num_clusters % 32 || num_clusters < 32 || num_queries < 0) return SBSA_ERR_ARG;
   int64_t bound = (int64_t)num_queries * num_kv_heads * num_clusters;
   if (qvals_cap < bound) return SBSA_ERR_CAPACITY;
-  int n = num_kv_heads * num_clusters;
-  hipLaunchKernelGGL(rev_pass_kernel, dim3(n), dim3(256), 0, stream, 0, qmask, num_queries,
-                     num_kv_heads, num_clusters, nvis, rev_counts, rev_indptr, qvals, qrank);
-  hipLaunchKernelGGL(rev_scan_kernel, dim3(1), dim3(1024), 0, stream, rev_counts, n, rev_indptr, nnz);
-  hipLaunchKernelGGL(rev_pass_kernel, dim3(n), dim3(256), 0, stream, 1, qmask, num_queries,
-                     num_kv_heads, num_clusters, nvis, rev_counts, rev_indptr, qvals, qrank);
+  launch_reverse_index(qmask, num_queries, num_kv_heads, num_clusters, nvis, rev_counts, rev_indptr, nnz, qvals,
+                       qrank, 1, ChunkBatch{}, stream);
   SBSA_CHECK_LAUNCH();
   return SBSA_OK;
 }
@@ -598,20 +655,48 @@ int sbsa_prefill_items(const int32_t* rev_counts, int num_kv_heads, int num_clus
                        hipStream_t stream) {
   if (!rev_counts || !items || !queue || queries_per_item < 1) return SBSA_ERR_ARG;
   if (!indptr || !nvis || !rev_indptr) return SBSA_ERR_ARG;
-  const int nloc = has_local ? (num_queries + queries_per_item - 1) / queries_per_item : 0;
-  const size_t lds = (size_t)(nloc * num_kv_heads + 3 * num_kv_heads * num_clusters) * 4;
-  if (lds > 150 * 1024) return SBSA_ERR_UNSUPPORTED;
-  static size_t configured = 0;
-  if (lds > configured) {
-    if (hipFuncSetAttribute((const void*)build_items_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
-                            (int)lds) != hipSuccess)
-      return SBSA_ERR_UNSUPPORTED;
-    configured = lds;
-  }
-  hipLaunchKernelGGL(build_items_kernel, dim3(1), dim3(1024), lds, stream, rev_counts, num_kv_heads,
-                     num_clusters, num_queries, queries_per_item, has_local, indptr, nvis, rev_indptr,
-                     (PrefillItem*)items, queue,
-                     items_cap, partials_cap);
+  const int rc = launch_items(rev_counts, num_kv_heads, num_clusters, num_queries, queries_per_item, has_local, indptr,
+                              nvis, rev_indptr, items, items_cap, partials_cap, partials_cap, queue, 1, ChunkBatch{},
+                              stream);
+  if (rc) return rc;
+  SBSA_CHECK_LAUNCH();
+  return SBSA_OK;
+}
+
+int sbsa_plan_chunks(const void* vectors, int64_t v_sq, int64_t v_sh, const void* codebooks, const int32_t* posting,
+                     int64_t width, const int32_t* indptr, const int32_t* sizes, int64_t first_pos, int num_queries,
+                     int chunk_queries, int num_q_heads, int num_kv_heads, int num_clusters, int dim,
+                     float inv_temperature, float beta, float target_tokens, int iters, int queries_per_item,
+                     int32_t* causal_sizes, int32_t* tokens, float* theta_out, int32_t* qmask, int32_t* rev_counts,
+                     int32_t* rev_indptr, int64_t* nnz, int32_t* qvals, int32_t* qrank, void* items, int64_t items_cap,
+                     int64_t partials_cap, int64_t last_partials_cap, int32_t* queues, hipStream_t stream) {
+  if (!posting || !indptr || !sizes || !causal_sizes || !qmask || !rev_counts || !rev_indptr || !nnz || !qvals ||
+      !qrank || !items || !queues)
+    return SBSA_ERR_ARG;
+  if (num_queries < 1 || chunk_queries < 1 || num_kv_heads < 1 || num_clusters < 64 || num_clusters % 64 ||
+      queries_per_item < 1)
+    return SBSA_ERR_ARG;
+  const int chunks = (num_queries + chunk_queries - 1) / chunk_queries;
+  const int ncl = num_kv_heads * num_clusters;
+  ChunkBatch cb;
+  cb.chunk_q = chunk_queries;
+  cb.total_q = num_queries;
+  cb.limit = chunk_queries;
+  cb.sizes = ncl;
+  cb.rev = ncl + 1;
+  cb.qvals = (int64_t)chunk_queries * ncl;
+  cb.items = items_cap;
+  hipLaunchKernelGGL(causal_sizes_kernel, dim3((ncl + 255) / 256, chunks), dim3(256), 0, stream, posting, width, indptr,
+                     sizes, num_kv_heads, num_clusters, first_pos, causal_sizes, cb);
+  int rc = sbsa_score_select(vectors, v_sq, v_sh, nullptr, codebooks, causal_sizes, ncl, num_clusters, num_queries,
+                             num_q_heads, num_kv_heads, num_clusters, dim, chunk_queries, inv_temperature, beta,
+                             target_tokens, iters, 0, nullptr, qmask, nullptr, tokens, nullptr, theta_out, stream);
+  if (rc) return rc;
+  launch_reverse_index(qmask, chunk_queries, num_kv_heads, num_clusters, causal_sizes, rev_counts, rev_indptr, nnz,
+                       qvals, qrank, chunks, cb, stream);
+  rc = launch_items(rev_counts, num_kv_heads, num_clusters, chunk_queries, queries_per_item, 1, indptr, causal_sizes,
+                    rev_indptr, items, items_cap, partials_cap, last_partials_cap, queues, chunks, cb, stream);
+  if (rc) return rc;
   SBSA_CHECK_LAUNCH();
   return SBSA_OK;
 }

@@ -4,7 +4,8 @@ semblo/vllm_plugin/fused_prefill.py seams, paper path: FA3 page 16, KV-outer).
   CausalSnapshot          cluster sizes at a position       (fused_prefill.py:44-135)
   fused_chunk_attention   dense prefix or select + KV-outer (fused_prefill.py:219-482),
                           also as its two halves: fused_chunk_plan (selection and
-                          reverse index) and fused_chunk_execute (the attention)
+                          reverse index) and fused_chunk_execute (the attention);
+                          fused_chunks_plan plans several chunks in one call
   fused_decode_attention  one query over the packed prompt  (fused_prefill.py:625-718)
 """
 from __future__ import annotations
@@ -16,7 +17,9 @@ import torch
 from . import _lib
 from .config import fitted_sink_tokens
 from .fused_select import theta_select_bitmask_flat
-from .kv_outer import dense_causal_attention, kv_outer_execute, kv_outer_plan
+from .kv_outer import (ITEM_INTS, QUEUE_INTS, QUEUE_OVERFLOW, KVOuterPlan, PartialsGuard,
+                       dense_causal_attention, kv_outer_execute, kv_outer_plan, partials_room, queries_per_item)
+from .trivial_router import trivial_router_vectors
 
 
 @dataclass(frozen=True)
@@ -132,6 +135,64 @@ def fused_chunk_plan(q_chunk: torch.Tensor, query_state, index, snapshot_state, 
         force_sink_bit(bitmask, qmask)
     kv = kv_outer_plan(qmask, causal_sizes, num_queries=q_count)
     return ChunkPlan(chunk_start, chunk_end, wstart, causal_sizes, tokens, kv, theta)
+
+
+# Most queries planned in one call: four of the paper's chunks (the routing vectors and the
+# reverse index's ranks of a group are held at once, 0.4 GB at 16 heads of 256 and 128 clusters).
+PLAN_GROUP_QUERIES = 32768
+
+
+def fused_chunks_plan(q_pre: torch.Tensor, index, first_pos: int, step: int, *, temperature: float, beta: float,
+                      target_tokens: int, iters: int = 16, guard: PartialsGuard | None = None,
+                      keep_theta: bool = False) -> list[ChunkPlan]:
+    """The plans, with their work lists, of consecutive sparse chunks of ``step`` queries
+    (the last one may be shorter): ``q_pre`` [n, Hq, D] from position ``first_pos``.  What
+    fused_chunk_plan and KVOuterPlan.prepare_work make per chunk, in one call for all of
+    them (sbsa_plan_chunks), for uniform mixture weights and no attention sink.  No host
+    read."""
+    n, hq, d = q_pre.shape
+    hkv, c = index.num_kv_heads, index.num_buckets
+    g = hq // hkv
+    dev = q_pre.device
+    chunks = -(-n // step)
+    qt = queries_per_item(g)
+    qns = [min(step, n - i * step) for i in range(chunks)]
+    rooms = {qn: partials_room(qn, hkv, c, g, d, q_pre.element_size(), guard) for qn in (qns[0], qns[-1])}
+    caps = [cap if capped else 0 for cap, capped in (rooms[qns[0]], rooms[qns[-1]])]
+    bound = max(1, *(_lib.query("sbsa_prefill_items_bound", rooms[qn][0], qn, hkv, c, qt) for qn in rooms))
+    vectors = trivial_router_vectors(q_pre, 1)
+
+    def ints(*shape):
+        return torch.empty(*shape, dtype=torch.int32, device=dev)
+
+    causal, counts, rev_indptr = ints(chunks, hkv, c), ints(chunks, hkv, c), ints(chunks, hkv * c + 1)
+    tokens, qmask, qrank = ints(n, hkv), ints(n, hkv, c // 32), ints(n, hkv, c)
+    qvals, items, queues = ints(chunks, step * hkv * c), ints(chunks, bound, ITEM_INTS), ints(chunks, QUEUE_INTS)
+    nnz = torch.empty(chunks, dtype=torch.int64, device=dev)
+    theta = torch.empty(n, hkv, dtype=torch.float32, device=dev) if keep_theta else None
+    _lib.call("sbsa_plan_chunks", _lib.ptr(vectors), vectors.stride(0), vectors.stride(1), _lib.ptr(index.codebooks),
+              _lib.ptr(index.posting_positions), index.posting_positions.shape[1], _lib.ptr(index.bucket_indptr),
+              _lib.ptr(index.bucket_sizes), int(first_pos), n, int(step), hq, hkv, c, d, 1.0 / float(temperature),
+              float(beta), float(target_tokens), int(iters), qt, _lib.ptr(causal), _lib.ptr(tokens), _lib.ptr(theta),
+              _lib.ptr(qmask), _lib.ptr(counts), _lib.ptr(rev_indptr), _lib.ptr(nnz), _lib.ptr(qvals),
+              _lib.ptr(qrank), _lib.ptr(items), bound, caps[0], caps[1], _lib.ptr(queues), _lib.stream(dev))
+    arrived = None
+    if any(caps):
+        # the overflow flags are final once the work lists are built
+        flags = torch.empty(chunks, dtype=torch.int32, pin_memory=True)
+        flags.copy_(queues[:, QUEUE_OVERFLOW], non_blocking=True)
+        arrived = torch.cuda.Event()
+        arrived.record()
+    plans = []
+    for i, qn in enumerate(qns):
+        a, b = i * step, i * step + qn
+        kv = KVOuterPlan(qmask[a:b], causal[i], qvals[i], counts[i], rev_indptr[i], nnz[i:i + 1], qrank[a:b])
+        cap, capped = rooms[qn]
+        kv.work = (cap, capped, items[i], queues[i], (arrived, flags[i:i + 1]) if capped else None)
+        start = first_pos + a
+        plans.append(ChunkPlan(start, start + qn - 1, start, causal[i], tokens[a:b], kv,
+                               theta[a:b] if keep_theta else None))
+    return plans
 
 
 def fused_chunk_execute(plan: ChunkPlan, q_chunk: torch.Tensor, index, nnz: int | None = None, *,

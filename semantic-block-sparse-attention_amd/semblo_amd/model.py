@@ -28,9 +28,10 @@ import torch
 from . import suffix_flush
 from .arena import DecodeArena
 from .attention_op import register_layer
-from .config import SembloRuntimeConfig
+from .config import SembloRuntimeConfig, fitted_sink_tokens
 from .fused_decode import fused_decode_step
-from .fused_prefill import CausalSnapshot, fused_chunk_execute, fused_chunk_plan
+from .fused_prefill import (PLAN_GROUP_QUERIES, CausalSnapshot, fused_chunk_execute, fused_chunk_plan,
+                            fused_chunks_plan)
 from .kv_outer import PartialsGuard
 from .kv_outer import dense_causal_attention
 from .state import ProductPostingIndex
@@ -309,44 +310,42 @@ class SembloAttention:
         side = self._build_stream(q.device)
         side.wait_event(inputs_ready)
         sparse = [(st, min(length, st + step)) for st in range(0, length, step) if st > cap]
-        # every sparse chunk's selection and reverse index on the build stream,
-        # each followed by an event; a chunk's attention waits for its own plan
-        # on the GPU only.  Its partial rows are sized by the capacity bound
-        # (kv_outer.partials_capacity), so the host reads nothing and every
+        # every sparse chunk's plan (selection, reverse index, work list) on the build
+        # stream, several chunks in one call followed by an event; a chunk's attention
+        # waits for its plan on the GPU only.  Its partial rows are sized by the capacity
+        # bound (kv_outer.partials_capacity), so the host reads nothing and every
         # chunk is enqueued at once.
-        plans, ready = [], []
         with torch.cuda.stream(side):
             index = self._ingest_prompt_kv(kp, kk, vv)
-            snapshot = CausalSnapshot(index)
-
-        def enqueue_plan(i):
-            st, en = sparse[i]
-            with torch.cuda.stream(side):
-                pl = fused_chunk_plan(q[st:en], self._query_state(qp[st:en]), index, snapshot, st,
-                                      en - 1, temperature=cfg.selection_temperature,
-                                      beta=cfg.bucket_size_penalty, target_tokens=self.target_tokens,
-                                      iters=cfg.iters, dense_prefix_x=cfg.dense_prefix_x,
-                                      keep_theta=self.plan_log is not None)
-                pl.record(self.plan_log)
-                # the chunk's work list too, here rather than on the main stream
-                # between two chunks' attention
-                pl.kv.prepare_work(q[st:en], index.num_kv_heads, index.bucket_indptr, guard)
-                ev = torch.cuda.Event()
-                ev.record(side)
-            plans.append(pl)
-            ready.append(ev)
-
         self.index = index
         # chunks whose partial rows were capped (kv_outer.partials_cap_bytes) are checked
         # once, after the last chunk is enqueued, and any that overflowed is run again;
         # each flag comes from the chunk's plan (copied when its work list is built), so
         # the check waits for the plans, not for the chunks' attention
         guard = PartialsGuard()
-        for i in range(len(sparse)):
-            enqueue_plan(i)
+        plans, ready = [], []
+        if sparse and fitted_sink_tokens():
+            self._plan_each(sparse, q, qp, index, side, guard, plans, ready)
+        else:
+            per_call = max(1, PLAN_GROUP_QUERIES // step)
+            for i in range(0, len(sparse), per_call):
+                group = sparse[i:i + per_call]
+                first, last = group[0][0], group[-1][1]
+                with torch.cuda.stream(side):
+                    pls = fused_chunks_plan(qp[first:last], index, first, step,
+                                            temperature=cfg.selection_temperature, beta=cfg.bucket_size_penalty,
+                                            target_tokens=self.target_tokens, iters=cfg.iters, guard=guard,
+                                            keep_theta=self.plan_log is not None)
+                    ev = torch.cuda.Event()
+                    ev.record(side)
+                for pl in pls:
+                    pl.record(self.plan_log)
+                plans += pls
+                ready += [ev] * len(pls)
         for i, (st, en) in enumerate(sparse):
             pl = plans[i]
-            main.wait_event(ready[i])
+            if i == 0 or ready[i] is not ready[i - 1]:
+                main.wait_event(ready[i])
             if i == 0:
                 for t in (index.codebooks, index.posting_positions, index.bucket_indptr,
                           index.bucket_sizes, index._inverse_positions, index.packed_kv):
@@ -367,6 +366,25 @@ class SembloAttention:
                 t.record_stream(main)
         self.adopt_index(index)
         return output
+
+    def _plan_each(self, sparse, q, qp, index, side, guard, plans, ready) -> None:
+        """The chunks' plans one by one (with an attention sink, which the plans of several
+        chunks in one call do not take)."""
+        cfg = self.runtime_config
+        snapshot = CausalSnapshot(index)
+        for st, en in sparse:
+            with torch.cuda.stream(side):
+                pl = fused_chunk_plan(q[st:en], self._query_state(qp[st:en]), index, snapshot, st,
+                                      en - 1, temperature=cfg.selection_temperature,
+                                      beta=cfg.bucket_size_penalty, target_tokens=self.target_tokens,
+                                      iters=cfg.iters, dense_prefix_x=cfg.dense_prefix_x,
+                                      keep_theta=self.plan_log is not None)
+                pl.record(self.plan_log)
+                pl.kv.prepare_work(q[st:en], index.num_kv_heads, index.bucket_indptr, guard)
+                ev = torch.cuda.Event()
+                ev.record(side)
+            plans.append(pl)
+            ready.append(ev)
 
     # -- decode -----------------------------------------------------------------
     def decode(self, positions, q_post, q_pre, k_post, v, output, k_pre=None) -> torch.Tensor:
