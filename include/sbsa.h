@@ -189,7 +189,10 @@ int sbsa_causal_sizes(const int32_t* posting, int64_t width, const int32_t* indp
  * each (head, cluster) with nvis > 0, the ascending query ids whose qmask has
  * it.  rev_counts [Hkv*C], rev_indptr [Hkv*C + 1], nnz (device int64), qvals
  * [qvals_cap >= Q*Hkv*C], qrank [Q, Hkv, C] (rank of q in the cluster's list,
- * written where selected).  Deterministic, no atomics. */
+ * written where selected).  Deterministic, no atomics.  With qvals_cap at least
+ * sbsa_reverse_index_ints(Q, Hkv, C), the room past the lists holds counts of the
+ * faster form. */
+int64_t sbsa_reverse_index_ints(int num_queries, int num_kv_heads, int num_clusters);
 int sbsa_reverse_index(const int32_t* qmask, int num_queries, int num_kv_heads, int num_clusters,
                        const int32_t* nvis, int32_t* rev_counts, int32_t* rev_indptr,
                        int64_t* nnz, int32_t* qvals, int64_t qvals_cap, int32_t* qrank,
@@ -235,7 +238,7 @@ int sbsa_prefill_items(const int32_t* rev_counts, int num_kv_heads, int num_clus
  * sbsa_reverse_index and sbsa_prefill_items, each in one set of launches for all
  * chunks.  first_pos: the first chunk's first position.  Outputs, one chunk after
  * another (n chunks): causal_sizes and rev_counts [n, Hkv, C], rev_indptr
- * [n, Hkv C + 1], nnz [n], qvals [n, chunk_queries Hkv C], items [n, items_cap],
+ * [n, Hkv C + 1], nnz [n], qvals [n, sbsa_reverse_index_ints(chunk_queries, Hkv, C)], items [n, items_cap],
  * queues [n, 32]; tokens [num_queries, Hkv], theta_out (or null) the same, qmask
  * [num_queries, Hkv, C/32], qrank [num_queries, Hkv, C].  partials_cap and
  * last_partials_cap as in sbsa_prefill_items, for the full chunks and the last. */

@@ -250,16 +250,9 @@ __global__ __launch_bounds__(256) void rev_pass_kernel(int pass, const int32_t* 
                                                        int32_t* __restrict__ rev_counts,
                                                        const int32_t* __restrict__ rev_indptr,
                                                        int32_t* __restrict__ qvals,
-                                                       int32_t* __restrict__ qrank, ChunkBatch cb) {
+                                                       int32_t* __restrict__ qrank) {
   __shared__ int wcnt[4];
   const int hc = blockIdx.x;
-  Q = cb.queries(Q);
-  qmask += (int64_t)blockIdx.y * cb.chunk_q * hkv * (C / 32);
-  nvis += blockIdx.y * cb.sizes;
-  rev_counts += blockIdx.y * cb.sizes;
-  rev_indptr += blockIdx.y * cb.rev;
-  qvals += blockIdx.y * cb.qvals;
-  qrank += (int64_t)blockIdx.y * cb.chunk_q * hkv * C;
   const int h = hc / C, c = hc % C;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int W = C / 32;
@@ -287,13 +280,131 @@ __global__ __launch_bounds__(256) void rev_pass_kernel(int pass, const int32_t* 
   if (pass == 0 && threadIdx.x == 0) rev_counts[hc] = run;
 }
 
+// The same in segments of REV_SEG queries, given scratch for a count per (segment,
+// head, cluster): a block takes one head's clusters over one segment and reads each
+// mask word once, where rev_pass_kernel's block walks all queries for one cluster (32
+// blocks re-read each word).  Pass 0 counts per segment; the scan below turns the
+// counts into each segment's first rank; pass 1 writes the lists.  One MI355X, 8192
+// queries, 4 heads, 128 clusters: 2 x 25 -> REV_FIGURES us for the two passes.
+constexpr int REV_SEG = 256;
+
+__global__ __launch_bounds__(REV_SEG) void rev_segment_kernel(int pass, const int32_t* __restrict__ qmask, int Q,
+                                                              int hkv, int C, const int32_t* __restrict__ nvis,
+                                                              int32_t* __restrict__ seg,
+                                                              const int32_t* __restrict__ rev_indptr,
+                                                              int32_t* __restrict__ qvals,
+                                                              int32_t* __restrict__ qrank, ChunkBatch cb) {
+  extern __shared__ int s_count[];     // [4 waves][C]: this wave's entries, then its first rank
+  const int h = blockIdx.z;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int W = C / 32;
+  Q = cb.queries(Q);
+  qmask += (int64_t)blockIdx.y * cb.chunk_q * hkv * W;
+  nvis += blockIdx.y * cb.sizes + h * C;
+  seg += blockIdx.y * cb.qvals + ((int64_t)blockIdx.x * hkv + h) * C;
+  rev_indptr += blockIdx.y * cb.rev + h * C;
+  qvals += blockIdx.y * cb.qvals;
+  qrank += (int64_t)blockIdx.y * cb.chunk_q * hkv * C;
+  const int q = blockIdx.x * REV_SEG + threadIdx.x;
+  const int32_t* words = qmask + ((int64_t)q * hkv + h) * W;
+  auto live_word = [&](int w) -> uint32_t {
+    const uint32_t live = (uint32_t)__ballot(lane < 32 && nvis[w * 32 + (lane & 31)] > 0);
+    return q < Q ? (uint32_t)words[w] & live : 0u;
+  };
+  int* mine = s_count + wave * C;
+  for (int w = 0; w < W; ++w) {
+    const uint32_t m = live_word(w);
+    int n = 0;
+#pragma unroll
+    for (int b = 0; b < 32; ++b) {
+      const int k = __popcll(__ballot((m >> b) & 1u));
+      if (lane == b) n = k;
+    }
+    if (lane < 32) mine[w * 32 + lane] = n;
+  }
+  __syncthreads();
+  if (pass == 0) {
+    for (int c = threadIdx.x; c < C; c += REV_SEG)
+      seg[c] = s_count[c] + s_count[C + c] + s_count[2 * C + c] + s_count[3 * C + c];
+    return;
+  }
+  for (int c = threadIdx.x; c < C; c += REV_SEG) {
+    int rank = seg[c];
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      const int n = s_count[v * C + c];
+      s_count[v * C + c] = rank;
+      rank += n;
+    }
+  }
+  __syncthreads();
+  const uint64_t below = (1ull << lane) - 1;
+  for (int w = 0; w < W; ++w) {
+    const uint32_t m = live_word(w);
+#pragma unroll 4
+    for (int b = 0; b < 32; ++b) {
+      const uint64_t ball = __ballot((m >> b) & 1u);
+      if ((m >> b) & 1u) {
+        const int c = w * 32 + b;
+        const int rank = mine[c] + __popcll(ball & below);
+        qvals[rev_indptr[c] + rank] = q;
+        qrank[((int64_t)q * hkv + h) * C + c] = rank;
+      }
+    }
+  }
+}
+
+// The segments' counts of each (head, cluster) into first ranks, their sum into
+// counts, then the exclusive scan of the sums (one block per chunk).
+__global__ __launch_bounds__(1024) void rev_segment_scan_kernel(int32_t* __restrict__ seg, int Q, int n,
+                                                                int32_t* __restrict__ counts,
+                                                                int32_t* __restrict__ indptr,
+                                                                int64_t* __restrict__ nnz, ChunkBatch cb) {
+  seg += blockIdx.y * cb.qvals;
+  counts += blockIdx.y * cb.sizes;
+  indptr += blockIdx.y * cb.rev;
+  const int segments = (cb.queries(Q) + REV_SEG - 1) / REV_SEG;
+  __shared__ int wsum[16];
+  __shared__ int carry;
+  if (threadIdx.x == 0) carry = 0;
+  __syncthreads();
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  for (int base = 0; base < n; base += 1024) {
+    const int i = base + threadIdx.x;
+    int v = 0;
+    if (i < n) {
+      for (int k0 = 0; k0 < segments; k0 += 8) {
+        int at[8];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) at[k] = k0 + k < segments ? seg[(int64_t)(k0 + k) * n + i] : 0;
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+          if (k0 + k < segments) seg[(int64_t)(k0 + k) * n + i] = v;
+          v += at[k];
+        }
+      }
+      counts[i] = v;
+    }
+    const int incl = wave_incl_scan(v);
+    if (lane == 63) wsum[wave] = incl;
+    __syncthreads();
+    int off = carry;
+    for (int w = 0; w < wave; ++w) off += wsum[w];
+    if (i < n) indptr[i] = off + incl - v;
+    __syncthreads();
+    if (threadIdx.x == 1023) carry = off + incl;
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) {
+    indptr[n] = carry;
+    nnz[blockIdx.y] = carry;
+  }
+}
+
 // Exclusive scan of the Hkv*C counts (one block), total into rev_indptr[n].
 __global__ __launch_bounds__(1024) void rev_scan_kernel(const int32_t* __restrict__ counts, int n,
                                                         int32_t* __restrict__ indptr,
-                                                        int64_t* __restrict__ nnz, ChunkBatch cb) {
-  counts += blockIdx.y * cb.sizes;
-  indptr += blockIdx.y * cb.rev;
-  nnz += blockIdx.y;
+                                                        int64_t* __restrict__ nnz) {
   __shared__ int wsum[16];
   __shared__ int carry;
   if (threadIdx.x == 0) carry = 0;
@@ -470,44 +581,48 @@ __global__ __launch_bounds__(1024) void build_items_kernel(const int32_t* __rest
     }
     __syncthreads();
   }
-  // expansion: one thread per source writes its items
-  for (int s = threadIdx.x; s < nsrc; s += 1024) {
+  // expansion: a thread per window tile, then a wave per cluster source (its
+  // lanes write the items side by side)
+  for (int s = threadIdx.x; s < nloc * hkv; s += 1024) {
+    const ItemSource si = item_source(rev_counts, s_order, s, nloc, hkv, C, Qc, QT);
+    if (s_first[s] < cap) items[s_first[s]] = PrefillItem{si.h, si.c, si.qb, si.qn, 0, 0, 0, 0};
+  }
+  for (int s = nloc * hkv + wave; s < nsrc; s += 16) {
     const ItemSource si = item_source(rev_counts, s_order, s, nloc, hkv, C, Qc, QT);
     if (!si.n) continue;
-    int64_t f0 = s_first[s];
-    int64_t rel = 0;
-    int ent = 0, row = 0, nk = 0;
-    if (si.c >= 0) {
-      nk = nvis[si.h * C + si.c];
-      ent = rev_indptr[si.h * C + si.c];
-      row = indptr[si.h * (C + 1) + si.c];
-    }
-    for (int j = 0; j < si.n; ++j, ++rel) {
-      const int64_t pos = f0 + rel;
-      if (pos >= cap) break;
-      const int qb = si.c >= 0 ? j * QT : si.qb;
-      const int qn = si.c >= 0 ? min(QT, si.qn - qb) : si.qn;
-      PrefillItem it{si.h, si.c, qb, qn, 0, 0, 0, 0};
-      if (si.c >= 0) {
-        it.nkeys = nk;
-        it.entry0 = ent + qb;
-        it.row0 = row;
-      }
-      items[pos] = it;
-    }
+    const int64_t f0 = s_first[s];
+    const int e = si.h * C + si.c;
+    const int nk = nvis[e], ent = rev_indptr[e], row = indptr[si.h * (C + 1) + si.c];
+    for (int j = lane; j < si.n; j += 64)
+      if (f0 + j < cap) items[f0 + j] = PrefillItem{si.h, si.c, j * QT, min(QT, si.qn - j * QT), nk, ent + j * QT, row, 0};
   }
 }
 
 
+int64_t rev_scratch(int num_queries, int ncl) { return (int64_t)((num_queries + REV_SEG - 1) / REV_SEG) * ncl; }
+
+// With scratch: the segment kernels (any number of chunks); without: a block per
+// (head, cluster) over all queries (one chunk).
 void launch_reverse_index(const int32_t* qmask, int num_queries, int hkv, int C, const int32_t* nvis,
                           int32_t* rev_counts, int32_t* rev_indptr, int64_t* nnz, int32_t* qvals, int32_t* qrank,
-                          int chunks, const ChunkBatch& cb, hipStream_t stream) {
+                          int32_t* scratch, int chunks, const ChunkBatch& cb, hipStream_t stream) {
   const int n = hkv * C;
-  hipLaunchKernelGGL(rev_pass_kernel, dim3(n, chunks), dim3(256), 0, stream, 0, qmask, num_queries, hkv, C, nvis,
-                     rev_counts, rev_indptr, qvals, qrank, cb);
-  hipLaunchKernelGGL(rev_scan_kernel, dim3(1, chunks), dim3(1024), 0, stream, rev_counts, n, rev_indptr, nnz, cb);
-  hipLaunchKernelGGL(rev_pass_kernel, dim3(n, chunks), dim3(256), 0, stream, 1, qmask, num_queries, hkv, C, nvis,
-                     rev_counts, rev_indptr, qvals, qrank, cb);
+  if (scratch && num_queries > 0) {
+    const dim3 grid((num_queries + REV_SEG - 1) / REV_SEG, chunks, hkv);
+    const size_t lds = (size_t)4 * C * sizeof(int);
+    hipLaunchKernelGGL(rev_segment_kernel, grid, dim3(REV_SEG), lds, stream, 0, qmask, num_queries, hkv, C, nvis,
+                       scratch, rev_indptr, qvals, qrank, cb);
+    hipLaunchKernelGGL(rev_segment_scan_kernel, dim3(1, chunks), dim3(1024), 0, stream, scratch, num_queries, n,
+                       rev_counts, rev_indptr, nnz, cb);
+    hipLaunchKernelGGL(rev_segment_kernel, grid, dim3(REV_SEG), lds, stream, 1, qmask, num_queries, hkv, C, nvis,
+                       scratch, rev_indptr, qvals, qrank, cb);
+    return;
+  }
+  hipLaunchKernelGGL(rev_pass_kernel, dim3(n), dim3(256), 0, stream, 0, qmask, num_queries, hkv, C, nvis,
+                     rev_counts, rev_indptr, qvals, qrank);
+  hipLaunchKernelGGL(rev_scan_kernel, dim3(1), dim3(1024), 0, stream, rev_counts, n, rev_indptr, nnz);
+  hipLaunchKernelGGL(rev_pass_kernel, dim3(n), dim3(256), 0, stream, 1, qmask, num_queries, hkv, C, nvis,
+                     rev_counts, rev_indptr, qvals, qrank);
 }
 
 int launch_items(const int32_t* rev_counts, int hkv, int C, int num_queries, int queries_per_item, int has_local,
@@ -627,6 +742,12 @@ int sbsa_causal_sizes(const int32_t* posting, int64_t width, const int32_t* indp
   return SBSA_OK;
 }
 
+int64_t sbsa_reverse_index_ints(int num_queries, int num_kv_heads, int num_clusters) {
+  if (num_queries < 0 || num_kv_heads < 1 || num_clusters < 1) return 0;
+  const int64_t ncl = (int64_t)num_kv_heads * num_clusters;
+  return num_queries * ncl + rev_scratch(num_queries, (int)ncl);
+}
+
 int sbsa_reverse_index(const int32_t* qmask, int num_queries, int num_kv_heads, int num_clusters,
                        const int32_t* nvis, int32_t* rev_counts, int32_t* rev_indptr,
                        int64_t* nnz, int32_t* qvals, int64_t qvals_cap, int32_t* qrank,
@@ -635,8 +756,11 @@ int sbsa_reverse_index(const int32_t* qmask, int num_queries, int num_kv_heads, 
   if (num_clusters % 32 || num_clusters < 32 || num_queries < 0) return SBSA_ERR_ARG;
   int64_t bound = (int64_t)num_queries * num_kv_heads * num_clusters;
   if (qvals_cap < bound) return SBSA_ERR_CAPACITY;
+  // room past the lists holds the segments' counts
+  int32_t* scratch =
+      qvals_cap >= bound + rev_scratch(num_queries, num_kv_heads * num_clusters) ? qvals + bound : nullptr;
   launch_reverse_index(qmask, num_queries, num_kv_heads, num_clusters, nvis, rev_counts, rev_indptr, nnz, qvals,
-                       qrank, 1, ChunkBatch{}, stream);
+                       qrank, scratch, 1, ChunkBatch{}, stream);
   SBSA_CHECK_LAUNCH();
   return SBSA_OK;
 }
@@ -684,7 +808,8 @@ int sbsa_plan_chunks(const void* vectors, int64_t v_sq, int64_t v_sh, const void
   cb.limit = chunk_queries;
   cb.sizes = ncl;
   cb.rev = ncl + 1;
-  cb.qvals = (int64_t)chunk_queries * ncl;
+  const int64_t lists = (int64_t)chunk_queries * ncl;
+  cb.qvals = lists + rev_scratch(chunk_queries, ncl);
   cb.items = items_cap;
   hipLaunchKernelGGL(causal_sizes_kernel, dim3((ncl + 255) / 256, chunks), dim3(256), 0, stream, posting, width, indptr,
                      sizes, num_kv_heads, num_clusters, first_pos, causal_sizes, cb);
@@ -693,7 +818,7 @@ int sbsa_plan_chunks(const void* vectors, int64_t v_sq, int64_t v_sh, const void
                              target_tokens, iters, 0, nullptr, qmask, nullptr, tokens, nullptr, theta_out, stream);
   if (rc) return rc;
   launch_reverse_index(qmask, chunk_queries, num_kv_heads, num_clusters, causal_sizes, rev_counts, rev_indptr, nnz,
-                       qvals, qrank, chunks, cb, stream);
+                       qvals, qrank, qvals + lists, chunks, cb, stream);
   rc = launch_items(rev_counts, num_kv_heads, num_clusters, chunk_queries, queries_per_item, 1, indptr, causal_sizes,
                     rev_indptr, items, items_cap, partials_cap, last_partials_cap, queues, chunks, cb, stream);
   if (rc) return rc;

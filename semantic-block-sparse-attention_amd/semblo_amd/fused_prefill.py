@@ -167,7 +167,8 @@ def fused_chunks_plan(q_pre: torch.Tensor, index, first_pos: int, step: int, *, 
 
     causal, counts, rev_indptr = ints(chunks, hkv, c), ints(chunks, hkv, c), ints(chunks, hkv * c + 1)
     tokens, qmask, qrank = ints(n, hkv), ints(n, hkv, c // 32), ints(n, hkv, c)
-    qvals, items, queues = ints(chunks, step * hkv * c), ints(chunks, bound, ITEM_INTS), ints(chunks, QUEUE_INTS)
+    qvals = ints(chunks, _lib.query("sbsa_reverse_index_ints", step, hkv, c))
+    items, queues = ints(chunks, bound, ITEM_INTS), ints(chunks, QUEUE_INTS)
     nnz = torch.empty(chunks, dtype=torch.int64, device=dev)
     theta = torch.empty(n, hkv, dtype=torch.float32, device=dev) if keep_theta else None
     _lib.call("sbsa_plan_chunks", _lib.ptr(vectors), vectors.stride(0), vectors.stride(1), _lib.ptr(index.codebooks),

@@ -49,7 +49,8 @@ def build_reverse_index(qmask: torch.Tensor, live: torch.Tensor, *, num_queries:
     counts = torch.empty(hkv, c, dtype=torch.int32, device=dev)
     indptr = torch.empty(hkv * c + 1, dtype=torch.int32, device=dev)
     nnz = torch.empty(1, dtype=torch.int64, device=dev)
-    cap = max(num_queries * hkv * c, 1)
+    # the lists' bound, and room behind them for the kernels' counts
+    cap = max(_lib.query("sbsa_reverse_index_ints", num_queries, hkv, c), 1)
     qvals = torch.empty(cap, dtype=torch.int32, device=dev)
     qrank = torch.empty(num_queries, hkv, c, dtype=torch.int32, device=dev)
     live32 = live if live.dtype == torch.int32 and live.is_contiguous() else live.to(torch.int32).contiguous()
@@ -95,10 +96,32 @@ def kv_outer_attention(q: torch.Tensor, packed_kv: torch.Tensor, qmask: torch.Te
     if k_loc.stride() != v_loc.stride():
         raise ValueError("the window's K and V must share a layout")
     plan = kv_outer_plan(qmask, causal_sizes, num_queries=qn)
-    nnz = int(plan.nnz_d.item())                  # the one host read of the chunk
-    return kv_outer_execute(q, packed_kv, plan, nnz, bucket_indptr, sm_scale=sm_scale,
-                            local_kv=local_kv, chunk_start=chunk_start, wstart=wstart, out=out,
-                            want_stats=want_stats, grid=grid, timing=timing)
+    # the one host read of the chunk, the partial count: copied behind the reverse index and
+    # read once the attention is enqueued, whose partial rows are sized by the bound known on
+    # the host, so the GPU does not wait for the host in between
+    count = torch.empty(1, dtype=torch.int64, pin_memory=True)
+    count.copy_(plan.nnz_d, non_blocking=True)
+    counted = torch.cuda.Event()
+    counted.record()
+    capped = _CappedChunk()
+    out, stats = kv_outer_execute(q, packed_kv, plan, None, bucket_indptr, sm_scale=sm_scale,
+                                  local_kv=local_kv, chunk_start=chunk_start, wstart=wstart, out=out,
+                                  want_stats=want_stats, grid=grid, timing=timing, guard=capped)
+    counted.synchronize()
+    stats["partials"] = int(count[0])
+    if capped.rerun is not None and stats["partials"] > partials_room(qn, hkv, c, g, d, q.element_size())[0]:
+        capped.rerun()
+    return out, stats
+
+
+class _CappedChunk:
+    """Stands in for a PartialsGuard where the caller reads the partial count itself."""
+
+    cap_entries = 0
+    rerun = None
+
+    def watch(self, queue, rerun, arrived=None) -> None:
+        self.rerun = rerun
 
 
 class KVOuterPlan:

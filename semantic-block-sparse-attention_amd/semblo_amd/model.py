@@ -22,6 +22,7 @@ one token starts a new request.
 from __future__ import annotations
 
 import os
+import threading
 
 import torch
 
@@ -36,6 +37,14 @@ from .kv_outer import PartialsGuard
 from .kv_outer import dense_causal_attention
 from .state import ProductPostingIndex
 from .trivial_router import trivial_router_vectors
+
+
+# Most queries of one dense launch beside the index build: the work list of 65536 queries fits the
+# 150 KB its builder takes for up to 8 KV heads.
+DENSE_LAUNCH_QUERIES = 65536
+
+
+_BUILD_STREAMS = threading.local()
 
 
 class SembloQueryState:
@@ -151,12 +160,14 @@ class SembloAttention:
         return index
 
     def _build_stream(self, device) -> torch.cuda.Stream:
-        """The stream the index is built on while the dense chunks run (default priority)."""
-        st = getattr(self, "_side_stream", None)
-        if st is None or st.device != torch.device(device):
-            st = torch.cuda.Stream(device=device)
-            self._side_stream = st
-        return st
+        """The stream the index is built on while the dense chunks run (default priority): one
+        per device and host thread, so that a new layer's build finds the memory that the
+        earlier layers' builds left to the stream (a stream of its own starts with none)."""
+        streams = _BUILD_STREAMS.__dict__.setdefault("by_device", {})
+        device = torch.device(device)
+        if device not in streams:
+            streams[device] = torch.cuda.Stream(device=device)
+        return streams[device]
 
     def begin_token_outer_prefill(self, tokens, chunk: int, **kw):
         """A token-order prefill session of a prompt (its length, or its positions as
@@ -299,12 +310,16 @@ class SembloAttention:
         main = torch.cuda.current_stream(q.device)
         inputs_ready = torch.cuda.Event()
         inputs_ready.record(main)
-        for start in range(0, min(length, cap + 1), step):
-            end = min(length, start + step)
+        # Several chunks to a launch: a chunk is rows of a longer one (the same arithmetic per
+        # row), and the launch's items, longest first, fill its tail.  grid -1: with room for
+        # the build's kernels on every compute unit.
+        dense_end = min(length, -(-min(length, cap + 1) // step) * step)
+        per_launch = max(1, DENSE_LAUNCH_QUERIES // step) * step
+        for start in range(0, dense_end, per_launch):
+            end = min(dense_end, start + per_launch)
             if timing is not None:
                 n = end - start
                 timing.add_flops(4.0 * self.head_dim * self.num_heads * (n * (start + 1) + n * (n - 1) // 2))
-            # grid -1: with room for the build's kernels on every compute unit
             dense_causal_attention(q[start:end], kk, vv, sm_scale=self.scaling, chunk_start=start,
                                    out=out[start:end], grid=-1, timing=timing)
         side = self._build_stream(q.device)
