@@ -132,7 +132,7 @@ int sbsa_bucket_layout(const int32_t* assign, int64_t length, int num_clusters, 
  * this 32-bit seed (torch's CPU randperm draws the same numbers): per fit the
  * sample [fit_n] (key rows), the initial rows [C] and the restart rows
  * [ahead][C] (sample rows), then each fit's head; sbsa_kmeans_draw_ints
- * entries in all.  length < 2^27.
+ * entries in all.  length < 2^27.  scratch: sbsa_kmeans_draw_scratch_ints.
  * sbsa_kmeans_fit: keys [length, heads, dim] bf16 at strides ld_k, ld_h; draws
  * on the device; sizes [heads, C], indptr [heads, C+1], posting
  * [heads, posting_cap], inverse [heads, length], codebooks
@@ -141,8 +141,9 @@ int sbsa_bucket_layout(const int32_t* assign, int64_t length, int num_clusters, 
  * head and those after it are not valid.  dim in {64, 128, 256}, rows 16-byte
  * aligned, the workspace 256-byte aligned. */
 int64_t sbsa_kmeans_draw_ints(int64_t fit_n, int heads, int num_clusters, int ahead);
+int64_t sbsa_kmeans_draw_scratch_ints(int64_t length, int64_t fit_n, int heads, int ahead);
 int sbsa_kmeans_draws(uint32_t seed, int64_t length, int64_t fit_n, int heads, int num_clusters, int ahead,
-                      int32_t* out);
+                      int32_t* out, int32_t* scratch);
 size_t sbsa_kmeans_fit_workspace_bytes(int64_t length, int64_t fit_n, int heads, int num_clusters, int dim,
                                        int ahead, int iters);
 int sbsa_kmeans_fit(const void* keys, int64_t length, int64_t ld_k, int64_t ld_h, int heads, int dim,

@@ -12,10 +12,6 @@
 //   state.py:950-997               pack_prompt_kv
 #include "sbsa_common.h"
 
-#include <atomic>
-#include <thread>
-#include <vector>
-
 namespace {
 
 // ---------------------------------------------------------------- S0 -------
@@ -1078,50 +1074,39 @@ extern "C" int64_t sbsa_kmeans_draw_ints(int64_t fit_n, int heads, int num_clust
   return (int64_t)num_fits(heads, ahead) * (fit_n + (int64_t)(1 + ahead) * num_clusters + 1);
 }
 
+// A head takes length - 1 words, fit_n - 1, and fit_n - 1 per restart; whole blocks of words.
+static int64_t draw_words(int64_t length, int64_t fit_n, int heads, int ahead) {
+  const int64_t most = heads * (length + fit_n - 2) + (int64_t)ahead * heads * (fit_n - 1);
+  return (most + 623) / 624 * 624;
+}
+
+extern "C" int64_t sbsa_kmeans_draw_scratch_ints(int64_t length, int64_t fit_n, int heads, int ahead) {
+  if (length < 1 || fit_n < 1 || heads < 1 || ahead < 1) return 0;
+  return draw_words(length, fit_n, heads, ahead) + length;
+}
+
 extern "C" int sbsa_kmeans_draws(uint32_t seed, int64_t length, int64_t fit_n, int heads, int num_clusters, int ahead,
-                                 int32_t* out) {
-  if (!out || !fit_shape_ok(length, fit_n, heads, num_clusters, 64, ahead, 1) || length >= (1ll << 27))
+                                 int32_t* out, int32_t* scratch) {
+  if (!out || !scratch || !fit_shape_ok(length, fit_n, heads, num_clusters, 64, ahead, 1) || length >= (1ll << 27))
     return SBSA_ERR_ARG;
-  try {
-    // a head takes length - 1 words, fit_n - 1, and fit_n - 1 per restart
-    const int64_t head_words = (length - 1) + (fit_n - 1);
-    const int64_t most = heads * head_words + (int64_t)ahead * heads * (fit_n - 1);
-    std::vector<uint32_t> words((size_t)(most + 623) / 624 * 624 + 624);
-    Mt19937 mt(seed);
-    for (size_t i = 0; i + 624 <= words.size(); i += 624) mt.block(words.data() + i);
-    const int64_t set = fit_n + (int64_t)(1 + ahead) * num_clusters;
-    const int fits = num_fits(heads, ahead);
-    for (int h = 0, fit = 0; h < heads; ++h)
-      for (int r = 0; r <= ahead * h; ++r) out[fits * set + fit++] = h;
-    // the fits' draws are independent of each other: shared out to a few threads
-    constexpr int THREADS = 4;
-    std::vector<int32_t> ident((size_t)length * THREADS);
-    std::atomic<int> next{0};
-    auto work = [&](int thread) {
-      int32_t* id = ident.data() + (size_t)length * thread;
-      for (int64_t i = 0; i < length; ++i) id[i] = (int32_t)i;
-      for (int fit = next++; fit < fits; fit = next++) {
-        const int h = out[fits * set + fit];
-        const int r = fit - (h + ahead * (h * (h - 1) / 2));
-        const uint32_t* w = words.data() + h * head_words + r * (fit_n - 1);
-        int32_t* at = out + fit * set;
-        permutation_prefix(w, length, fit_n, id, at);
-        w += length - 1;
-        for (int k = 0; k <= ahead; ++k)      // the initial rows, then the restarts'
-          permutation_prefix(w + k * (fit_n - 1), fit_n, num_clusters, id, at + fit_n + (int64_t)k * num_clusters);
-      }
-    };
-    std::vector<std::thread> others;
-    try {
-      for (int t = 1; t < THREADS && t < fits; ++t) others.emplace_back(work, t);
-    } catch (...) {
-      // fewer threads: the others take its share
+  const int64_t head_words = (length - 1) + (fit_n - 1), n_words = draw_words(length, fit_n, heads, ahead);
+  uint32_t* words = (uint32_t*)scratch;
+  Mt19937 mt(seed);
+  for (int64_t i = 0; i < n_words; i += 624) mt.block(words + i);
+  int32_t* ident = scratch + n_words;
+  for (int64_t i = 0; i < length; ++i) ident[i] = (int32_t)i;
+  const int64_t set = fit_n + (int64_t)(1 + ahead) * num_clusters;
+  int32_t* head_of = out + num_fits(heads, ahead) * set;
+  int32_t* at = out;
+  for (int h = 0; h < heads; ++h)
+    for (int r = 0; r <= ahead * h; ++r, at += set) {
+      const uint32_t* w = words + h * head_words + r * (fit_n - 1);
+      permutation_prefix(w, length, fit_n, ident, at);
+      w += length - 1;
+      for (int k = 0; k <= ahead; ++k)      // the initial rows, then the restarts'
+        permutation_prefix(w + k * (fit_n - 1), fit_n, num_clusters, ident, at + fit_n + (int64_t)k * num_clusters);
+      *head_of++ = h;
     }
-    work(0);
-    for (auto& t : others) t.join();
-  } catch (...) {
-    return SBSA_ERR_CAPACITY;
-  }
   return SBSA_OK;
 }
 

@@ -105,9 +105,13 @@ def _fit_batched(pk: torch.Tensor, *, seed: int, fit_n: int, c: int, iters: int,
     if ws_bytes == 0 or ws_bytes > BATCH_BYTES:
         return None
     n_draws = _lib.query("sbsa_kmeans_draw_ints", fit_n, hkv, c, RESTARTS_AHEAD)
-    host = torch.empty(n_draws, dtype=torch.int32, pin_memory=True)
-    _lib.call("sbsa_kmeans_draws", seed & 0xffffffff, length, fit_n, hkv, c, RESTARTS_AHEAD, host.data_ptr())
-    draws = host.to(dev, non_blocking=True)
+    # drawn into pinned memory, the draws' scratch behind them (memory the host allocator
+    # keeps: fresh pages would cost more than the draws)
+    n_scratch = _lib.query("sbsa_kmeans_draw_scratch_ints", length, fit_n, hkv, RESTARTS_AHEAD)
+    host = torch.empty(n_draws + n_scratch, dtype=torch.int32, pin_memory=True)
+    _lib.call("sbsa_kmeans_draws", seed & 0xffffffff, length, fit_n, hkv, c, RESTARTS_AHEAD, host.data_ptr(),
+              host[n_draws:].data_ptr())
+    draws = host[:n_draws].to(dev, non_blocking=True)
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
     cap = length + c * (align - 1)
     posting = torch.empty(hkv, cap, dtype=torch.int32, device=dev)

@@ -16,7 +16,9 @@ def test_draws_equal_torch_randperm(seed, length, fit_n, heads, c, ahead):
         pytest.skip("libsbsa.so is not built here")
     n = _lib.query("sbsa_kmeans_draw_ints", fit_n, heads, c, ahead)
     out = torch.empty(n, dtype=torch.int32)
-    _lib.call("sbsa_kmeans_draws", seed & 0xffffffff, length, fit_n, heads, c, ahead, out.data_ptr())
+    scratch = torch.empty(_lib.query("sbsa_kmeans_draw_scratch_ints", length, fit_n, heads, ahead), dtype=torch.int32)
+    _lib.call("sbsa_kmeans_draws", seed & 0xffffffff, length, fit_n, heads, c, ahead, out.data_ptr(),
+              scratch.data_ptr())
     fits = heads + ahead * (heads * (heads - 1) // 2)
     size = fit_n + (1 + ahead) * c
     assert n == fits * (size + 1)
@@ -44,6 +46,6 @@ def test_draws_refuse_bad_shapes():
         pytest.skip("libsbsa.so is not built here")
     lib = _lib.load()
     out = torch.empty(100000, dtype=torch.int32)
-    assert lib.sbsa_kmeans_draws(1, 100, 200, 1, 64, 2, out.data_ptr()) == 1      # sample larger than the keys
-    assert lib.sbsa_kmeans_draws(1, 200, 32, 1, 64, 2, out.data_ptr()) == 1       # fewer rows than clusters
-    assert lib.sbsa_kmeans_draws(1, 200, 100, 1, 64, 2, None) == 1
+    assert lib.sbsa_kmeans_draws(1, 100, 200, 1, 64, 2, out.data_ptr(), out.data_ptr()) == 1      # sample larger than the keys
+    assert lib.sbsa_kmeans_draws(1, 200, 32, 1, 64, 2, out.data_ptr(), out.data_ptr()) == 1       # fewer rows than clusters
+    assert lib.sbsa_kmeans_draws(1, 200, 100, 1, 64, 2, None, out.data_ptr()) == 1
