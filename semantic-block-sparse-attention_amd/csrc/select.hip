@@ -9,12 +9,21 @@
 //   kv_outer.py:41-173, 254-329 build_reverse_index
 #include "sbsa_common.h"
 
+#include <type_traits>
+
 namespace {
 
 // ------------------------------------------------------------- S2 + S3 -----
 // One block = QT queries x one KV head.  Rows of the score GEMM are
 // (query, component) pairs, R = QT * G of them; the four waves split the
 // clusters.  Scores live in LDS; each wave then selects for its queries.
+// Bound by the chains of a wave's selection (reductions over the lanes, the bisection's
+// ballots and counts), not by memory or the matrix units, so the row softmax is taken by
+// the query's own wave, all components' reductions side by side, and its weights stay in
+// registers: no second walk of the table and no block barrier before the selection.  One
+// MI355X, a call with its bitmask fill: C = 256, 8192 queries of 16 heads on 4, D = 256
+// 158 -> 117 us, C = 128 97 -> 76 us, C = 512 (8192 queries, 8 heads on 1, D = 128)
+// 127 -> 87 us, C = 1024 (2048 queries, 4 on 4, D = 256) 91 -> 78 us.
 struct SelectArgs {
   const bf16_t* vectors;   // [Q, Hq, D] routing vectors
   int64_t v_sq, v_sh;      // element strides
@@ -32,14 +41,16 @@ struct SelectArgs {
   float inv_temp, beta, target;
 };
 
-template <int D, int NK>
+// NK: clusters per lane at most; EXACT: C is 64 NK (64, 128, 256, 512, 1024), so that
+// the loops over a lane's clusters are straight-line code.
+template <int D, int NK, bool EXACT>
 __global__ __launch_bounds__(256) void score_select_kernel(SelectArgs a, int R) {
   constexpr int KS = D / 32;
   constexpr int LDQ = D + 8;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   bf16_t* sq = reinterpret_cast<bf16_t*>(smem);                      // [R][LDQ]
   float* ssc = reinterpret_cast<float*>(smem + (size_t)R * LDQ * 2);  // [R][C+1]
-  const int C = a.C, G = a.G;
+  const int C = EXACT ? 64 * NK : a.C, G = a.G;
   const int LDS_C = C + 1;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int h = blockIdx.y;
@@ -58,9 +69,19 @@ __global__ __launch_bounds__(256) void score_select_kernel(SelectArgs a, int R) 
   }
   __syncthreads();
 
-  // scores: each wave takes C/4 clusters (a multiple of 16)
+  // scores: each wave takes C/4 clusters (a multiple of 16); its rows' operands stay in
+  // registers over the clusters when they fit (R <= 32)
   const int cols_per_wave = C / 4;
   const bf16_t* cb = a.codebooks + (int64_t)h * 2 * C * half;
+  constexpr int RB = 2;
+  u32x4_t aop[RB][KS];
+  auto load_a = [&](int rb, u32x4_t (&v)[KS]) {
+#pragma unroll
+    for (int s = 0; s < KS; ++s)
+      v[s] = *reinterpret_cast<const u32x4_t*>(&sq[(rb * 16 + (lane & 15)) * LDQ + s * 32 + (lane >> 4) * 8]);
+  };
+#pragma unroll
+  for (int rb = 0; rb < RB; ++rb) load_a(min(rb, R / 16 - 1), aop[rb]);
   for (int cbk = 0; cbk < cols_per_wave / 16; ++cbk) {
     const int col0 = wave * cols_per_wave + cbk * 16;
     const int cc = col0 + (lane & 15);
@@ -71,38 +92,76 @@ __global__ __launch_bounds__(256) void score_select_kernel(SelectArgs a, int R) 
       int part = d / half;
       bop[s] = *reinterpret_cast<const u32x4_t*>(cb + ((int64_t)part * C + cc) * half + (d - part * half));
     }
-    for (int rb = 0; rb < R / 16; ++rb) {
+    auto score = [&](int rb, const u32x4_t (&v)[KS]) {
       f32x4_t acc = f32x4_t{0, 0, 0, 0};
 #pragma unroll
-      for (int s = 0; s < KS; ++s) {
-        u32x4_t aop = *reinterpret_cast<const u32x4_t*>(&sq[(rb * 16 + (lane & 15)) * LDQ + s * 32 + (lane >> 4) * 8]);
-        acc = mfma16x16x32(as_bf16x8(aop), as_bf16x8(bop[s]), acc);
-      }
+      for (int s = 0; s < KS; ++s) acc = mfma16x16x32(as_bf16x8(v[s]), as_bf16x8(bop[s]), acc);
 #pragma unroll
       for (int i = 0; i < 4; ++i) ssc[(rb * 16 + (lane >> 4) * 4 + i) * LDS_C + cc] = acc[i] * a.inv_temp;
+    };
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb)
+      if (rb < R / 16) score(rb, aop[rb]);
+    for (int rb = RB; rb < R / 16; ++rb) {
+      u32x4_t v[KS];
+      load_a(rb, v);
+      score(rb, v);
     }
   }
   __syncthreads();
 
-  // per row: lse over C, then w = exp(s - lse + logmix) in place (base-2
-  // hardware exp/log: about 1 ulp, far below the selection's near-tie margin)
+  // per row (query, component): lse over C, then each cluster's w = exp(s - lse +
+  // logmix) (base-2 hardware exp/log: about 1 ulp, far below the selection's near-tie
+  // margin).  The rows r0, r0 + step, .. of a call are taken together, so that their
+  // reductions overlap; v holds the lane's clusters, scores in and weights out.
   constexpr float LOG2E = 1.4426950408889634f;
-  for (int r = wave; r < R; r += 4) {
-    float* row = ssc + r * LDS_C;
-    float m = -INFINITY;
-    for (int c = lane; c < C; c += 64) m = fmaxf(m, row[c]);
-    m = wave_max_dpp(m);
-    float l = 0.f;
-    for (int c = lane; c < C; c += 64) l += __builtin_amdgcn_exp2f((row[c] - m) * LOG2E);
-    l = wave_sum_dpp(l);
-    int q = q0 + r / G, t = r % G;
-    float lm = 0.f;
-    if (a.logmix && q < a.Q) lm = a.logmix[(int64_t)q * a.Hq + h * G + t];
-    // log2 of exp(lm) / (sum exp(s))
-    const float off2 = (lm - m) * LOG2E - __builtin_amdgcn_logf(l);
-    for (int c = lane; c < C; c += 64) row[c] = __builtin_amdgcn_exp2f(__builtin_fmaf(row[c], LOG2E, off2));
+  auto softmax_rows = [&](auto rows, int r0, int step, auto& v) {
+    constexpr int N = decltype(rows)::value;
+    float m[N], l[N];
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      const float* row = ssc + (r0 + step * i) * LDS_C;
+      m[i] = -INFINITY;
+#pragma unroll
+      for (int k = 0; k < NK; ++k) {
+        v[i][k] = (64 * k < C) ? row[lane + 64 * k] : -INFINITY;
+        m[i] = fmaxf(m[i], v[i][k]);
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < N; ++i) m[i] = wave_max_dpp(m[i]);
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      l[i] = 0.f;
+#pragma unroll
+      for (int k = 0; k < NK; ++k)
+        if (64 * k < C) l[i] += __builtin_amdgcn_exp2f((v[i][k] - m[i]) * LOG2E);
+    }
+#pragma unroll
+    for (int i = 0; i < N; ++i) l[i] = wave_sum_dpp(l[i]);
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      const int r = r0 + step * i, q = q0 + r / G, t = r % G;
+      float lm = 0.f;
+      if (a.logmix && q < a.Q) lm = a.logmix[(int64_t)q * a.Hq + h * G + t];
+      // log2 of exp(lm) / (sum exp(s))
+      const float off2 = (lm - m[i]) * LOG2E - __builtin_amdgcn_logf(l[i]);
+#pragma unroll
+      for (int k = 0; k < NK; ++k) v[i][k] = __builtin_amdgcn_exp2f(__builtin_fmaf(v[i][k], LOG2E, off2));
+    }
+  };
+  // up to four components, the wave of a query takes their softmax itself (below);
+  // with more, the weights go back into the table first
+  if (G > 4) {
+    for (int r = wave; r < R; r += 4) {
+      float v[1][NK];
+      softmax_rows(std::integral_constant<int, 1>(), r, 0, v);
+#pragma unroll
+      for (int k = 0; k < NK; ++k)
+        if (64 * k < C) ssc[r * LDS_C + lane + 64 * k] = v[0][k];
+    }
+    __syncthreads();
   }
-  __syncthreads();
 
   // selection, one wave per query; lane holds clusters lane + 64k
   const int W = C / 32;
@@ -118,6 +177,32 @@ __global__ __launch_bounds__(256) void score_select_kernel(SelectArgs a, int R) 
     const int nk = C / 64;
     float hi = -INFINITY, lo = INFINITY;
     int live_total = 0;      // token counts: sizes sum to at most the prompt length
+    // each cluster's weight: the components' sum, in component order
+    float pw[NK];
+    auto weights = [&](auto g) {
+      float w[g.value][NK];
+      softmax_rows(g, qi * G, 1, w);
+#pragma unroll
+      for (int k = 0; k < NK; ++k) {
+        pw[k] = 0.f;
+#pragma unroll
+        for (int t = 0; t < g.value; ++t) pw[k] += w[t][k];
+      }
+    };
+    if (G == 4) {
+      weights(std::integral_constant<int, 4>());
+    } else if (G == 2) {
+      weights(std::integral_constant<int, 2>());
+    } else if (G == 1) {
+      weights(std::integral_constant<int, 1>());
+    } else {
+#pragma unroll
+      for (int k = 0; k < NK; ++k) {
+        pw[k] = 0.f;
+        if (64 * k < C)
+          for (int t = 0; t < G; ++t) pw[k] += ssc[(qi * G + t) * LDS_C + lane + 64 * k];
+      }
+    }
 #pragma unroll
     for (int k = 0; k < NK; ++k) {
       score[k] = NEG;
@@ -126,8 +211,7 @@ __global__ __launch_bounds__(256) void score_select_kernel(SelectArgs a, int R) 
       real_size[k] = 0.f;
       if (k < nk) {
         int c = lane + 64 * k;
-        float p = 0.f;
-        for (int t = 0; t < G; ++t) p += ssc[(qi * G + t) * LDS_C + c];
+        const float p = pw[k];
         if (a.prob_out) a.prob_out[((int64_t)q * a.Hkv + h) * C + c] = p;
         float rs = (float)sz[c];
         float s = (a.sink > 0 && c == 0) ? 0.f : rs;  // the sink is hidden from the search
@@ -154,8 +238,31 @@ __global__ __launch_bounds__(256) void score_select_kernel(SelectArgs a, int R) 
     const bool all_fit = (float)live_total < budget;
     const int bud_i = budget_count(budget);
     // two bisection steps per round: the first step's mid and both possible
-    // second mids are counted together (the same fp32 mids as one step at a time)
+    // second mids are counted together (the same fp32 mids as one step at a time).
+    // Once a mid has failed, the count reaches the budget at lo and not at hi; with
+    // one score left in [lo, hi), a mid between them reaches it exactly when it is
+    // not above that score, and the remaining steps need no counts.
+    bool failed = false;
     for (int it = 0; it < a.iters; it += 2) {
+      if (failed && it % 4 == 0) {
+        int inside = 0;
+        float last = NEG;
+#pragma unroll
+        for (int k = 0; k < NK; ++k) {
+          const bool in = score[k] >= lo && score[k] < hi;
+          inside += __popcll(__ballot(in));
+          last = in ? score[k] : last;
+        }
+        if (inside == 1) {
+          last = wave_max_dpp(last);
+          for (int j = it; j < a.iters; ++j) {
+            const float mid = (lo + hi) * 0.5f;
+            if (mid <= last) lo = mid;
+            else hi = mid;
+          }
+          break;
+        }
+      }
       const float m0 = (lo + hi) * 0.5f;
       const float m1 = (m0 + hi) * 0.5f;     // second mid if m0 reaches the budget
       const float m2 = (lo + m0) * 0.5f;     // second mid otherwise
@@ -171,10 +278,11 @@ __global__ __launch_bounds__(256) void score_select_kernel(SelectArgs a, int R) 
         lo = m0;
         if (it + 1 < a.iters) {
           if (c1 >= bud_i) lo = m1;
-          else hi = m1;
+          else hi = m1, failed = true;
         }
       } else {
         hi = m0;
+        failed = true;
         if (it + 1 < a.iters) {
           if (c2 >= bud_i) lo = m2;
           else hi = m2;
@@ -285,7 +393,7 @@ __global__ __launch_bounds__(256) void rev_pass_kernel(int pass, const int32_t* 
 // mask word once, where rev_pass_kernel's block walks all queries for one cluster (32
 // blocks re-read each word).  Pass 0 counts per segment; the scan below turns the
 // counts into each segment's first rank; pass 1 writes the lists.  One MI355X, 8192
-// queries, 4 heads, 128 clusters: 2 x 25 -> REV_FIGURES us for the two passes.
+// queries, 4 heads, 128 clusters: 2 x 25 -> 6.6 + 22.1 us for the two passes.
 constexpr int REV_SEG = 256;
 
 __global__ __launch_bounds__(REV_SEG) void rev_segment_kernel(int pass, const int32_t* __restrict__ qmask, int Q,
@@ -650,11 +758,11 @@ int launch_items(const int32_t* rev_counts, int hkv, int C, int num_queries, int
 // One instantiation per bound on the clusters a lane holds (C <= 64 NK).
 template <int D, int NK>
 int launch_select_nk(const SelectArgs& a, dim3 grid, size_t lds, int R, hipStream_t stream) {
-  if (lds > 64 * 1024 &&
-      hipFuncSetAttribute((const void*)score_select_kernel<D, NK>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                          (int)lds) != hipSuccess)
+  auto kernel = a.C == 64 * NK ? score_select_kernel<D, NK, true> : score_select_kernel<D, NK, false>;
+  if (lds > 64 * 1024 && hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                             (int)lds) != hipSuccess)
     return SBSA_ERR_UNSUPPORTED;
-  hipLaunchKernelGGL((score_select_kernel<D, NK>), grid, dim3(256), lds, stream, a, R);
+  hipLaunchKernelGGL(kernel, grid, dim3(256), lds, stream, a, R);
   return SBSA_OK;
 }
 template <int D>
@@ -663,6 +771,7 @@ int launch_select(const SelectArgs& a, dim3 grid, size_t lds, int R, hipStream_t
   if (nk <= 1) return launch_select_nk<D, 1>(a, grid, lds, R, stream);
   if (nk <= 2) return launch_select_nk<D, 2>(a, grid, lds, R, stream);
   if (nk <= 4) return launch_select_nk<D, 4>(a, grid, lds, R, stream);
+  if (nk <= 8) return launch_select_nk<D, 8>(a, grid, lds, R, stream);
   return launch_select_nk<D, 16>(a, grid, lds, R, stream);
 }
 
@@ -685,7 +794,8 @@ int sbsa_score_select(const void* vectors, int64_t v_sq, int64_t v_sh, const flo
   if (num_queries == 0) return SBSA_OK;
   // rows (query, component) per block: 32 keep a block's LDS near 50 KB at
   // C <= 256, so three blocks share a CU and hide each other's reduction
-  // chains (C = 256, 8192 queries: 373 us with 64 rows, 173 us with 32, 205 with 16)
+  // chains (C = 256, 8192 queries, with the softmax through the table: 373 us with
+  // 64 rows, 173 us with 32, 205 with 16)
   int R = (C <= 256) ? 32 : (C <= 512 ? 32 : 16);
   if (R < G) R = G;
   if (R % 16) R = 16;
