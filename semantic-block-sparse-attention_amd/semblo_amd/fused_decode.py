@@ -74,6 +74,9 @@ def fused_decode_step(layer, arena, *, q_post: torch.Tensor, q_pre: torch.Tensor
     if k_post is not None and v_states is not None:
         kk = k_post.reshape(hkv, d)
         vv = v_states.reshape(hkv, d)
+        # the step reads both with K's row stride
+        if (hkv > 1 and vv.stride(0) != kk.stride(0)) or kk.stride(-1) != 1 or vv.stride(-1) != 1:
+            raise ValueError("k_post and v_states need unit inner strides and one row stride")
         if k_pre is not None and getattr(arena, "suffix_kpre", None) is not None:
             kp = k_pre.reshape(hkv, d)
             if kp.stride(0) != kk.stride(0) or kp.stride(-1) != 1:
