@@ -294,6 +294,7 @@ __forceinline__ void raw_buffer_store(T v, rsrc_t r, int voffset, int soffset) {
 #define __builtin_amdgcn_logf(x) log2f(x)
 #define __builtin_amdgcn_s_waitcnt(x) emu::waitcnt((unsigned)(x))
 #define __builtin_amdgcn_sched_barrier(x) ((void)0)
+#define __builtin_amdgcn_s_setprio(x) ((void)0)
 #define __builtin_amdgcn_sched_group_barrier(a, b, c) ((void)0)
 #define __builtin_amdgcn_wave_barrier() emu::wave_sync()
 #define __builtin_amdgcn_fence(...) std::atomic_thread_fence(std::memory_order_seq_cst)
