@@ -211,18 +211,22 @@ __global__ __launch_bounds__(256, 1) void attn_items_kernel(AttnArgs a) {
   // the queues' sizes and offsets are read once, into LDS
   __shared__ int s_queue[16];
   if (threadIdx.x < 16) s_queue[threadIdx.x] = a.queue[threadIdx.x];
-  int pend = 0;
-  if (threadIdx.x == 0) pend = atomicAdd(&a.queue[16 + home], 1);
   __syncthreads();
   // The first 2 B positions of each segment (B = blocks per segment) are
   // paired statically: the block of rank i in its segment takes positions i
   // and 2 B - 1 - i.  Segments start with their longest items, so a pair
   // (long, short) evens out the blocks' first shares, which would otherwise
   // go by the order of the first atomic claims.  The later positions are
-  // claimed through the segment's counter.
+  // claimed through the segment's counter; a segment of no more than 2 B items has none,
+  // and its counter is not touched (see attn_pair_kernel).
   const int nstat = (gridDim.x % 8 == 0) ? 2 * (int)(gridDim.x / 8) : 0;
   const int srank = (int)(blockIdx.x >> 3);
-  int nclaims = 0;
+  int pend = 0, nclaims = 0;
+  auto request = [&]() {
+    while (probe < 8 && s_queue[(home + probe) & 7] <= nstat) ++probe;
+    if (probe < 8) pend = atomicAdd(&a.queue[16 + ((home + probe) & 7)], 1);
+  };
+  if (threadIdx.x == 0) request();
   // thread 0 only: the next item of this block's queue (stealing from the
   // other XCDs' queues once it is empty), -1 when every queue is
   auto claim = [&]() -> int {
@@ -230,18 +234,14 @@ __global__ __launch_bounds__(256, 1) void attn_items_kernel(AttnArgs a) {
       const int pos = nclaims++ == 0 ? srank : nstat - 1 - srank;
       if (pos < s_queue[home]) return s_queue[8 + home] + pos;
     }
-    int claimed = -1;
-    for (;;) {
-      const int x = (home + probe) & 7;
-      if (nstat + pend < s_queue[x]) {
-        claimed = s_queue[8 + x] + nstat + pend;
-        break;
-      }
-      if (++probe == 8) break;
-      pend = atomicAdd(&a.queue[16 + ((home + probe) & 7)], 1);
+    while (probe < 8) {
+      const int x = (home + probe) & 7, pos = nstat + pend;
+      const bool got = pos < s_queue[x];
+      if (!got) ++probe;
+      request();
+      if (got) return s_queue[8 + x] + pos;
     }
-    if (claimed >= 0) pend = atomicAdd(&a.queue[16 + ((home + probe) & 7)], 1);
-    return claimed;
+    return -1;
   };
   // Claims run two items ahead through two LDS slots, so reading one needs no
   // barrier: when an item starts, the next item's index (slot of parity i + 1)
@@ -778,11 +778,14 @@ __global__ __launch_bounds__(256, 2) void attn_pair_kernel(AttnArgs a) {
   // segment (B = blocks per XCD) are paired statically, a long item with a short
   // one; later positions come from the segment's counter, and from the other
   // segments' once it is empty.  The counter's atomic is issued at an item's end
-  // and read after the next item's first tile, when every load has landed.
+  // and read after the next item's first tile, when every load has landed.  A segment
+  // without later positions is passed by: in a call of few items, 512 blocks asking
+  // eight counters each were 46 us of atomics on the same lines (90 ns per block).
   const int nstat = (gridDim.x % 8 == 0) ? 2 * (int)(gridDim.x / 8) : 0;
   int pend = -1, nclaims = 0;
   auto request = [&]() {
-    if (threadIdx.x == 0 && pend < 0 && probe < 8) pend = atomicAdd(&a.queue[16 + ((home + probe) & 7)], 1);
+    if (threadIdx.x == 0 && pend < 0 && probe < 8 && s_queue[(home + probe) & 7] > nstat)
+      pend = atomicAdd(&a.queue[16 + ((home + probe) & 7)], 1);
   };
   auto claim = [&]() -> int {
     while (nclaims < 2 && nstat > 0) {
@@ -792,6 +795,7 @@ __global__ __launch_bounds__(256, 2) void attn_pair_kernel(AttnArgs a) {
     }
     for (; probe < 8; ++probe) {
       const int x = (home + probe) & 7;
+      if (s_queue[x] <= nstat) continue;
       if (pend < 0) pend = atomicAdd(&a.queue[16 + x], 1);
       const int pos = nstat + pend;
       pend = -1;
@@ -1314,20 +1318,32 @@ int launch_attn_kernel(AttnKernel kernel, int& auto_grid, const AttnArgs& a, int
   return SBSA_OK;
 }
 
-// Which form: two blocks per compute unit, unless the caller asks for room for
-// other streams' kernels (grid < 0): the one-block form then leaves registers and
-// LDS on every compute unit.  The layer asks for it for the dense chunks that run
-// beside its index build: the other form holds every register, so the build would
-// follow it (prefill of 32768: 5.5 ms with the one-block dense chunks, 6.8 with
-// these; of 131072: 42.1 and 42.7).  Alone, a dense chunk of 8192 queries at
-// 24576 takes 2967 us in the two-block form and 3458 in the other.  A window's
-// rows whose output offsets pass 31 bits go to the one-block form too.
+// Which form.  A caller that asks for room for other streams' kernels (grid < 0) gets the
+// one-block form, which leaves registers and LDS on every compute unit: the layer asks for
+// it for the dense chunks that run beside its index build (the other form holds every
+// register, so the build would follow it: prefill of 32768 5.5 ms with the one-block dense
+// chunks, 6.8 with these; of 131072 42.1 and 42.7).  An explicit grid gets the two-block form.
+// Otherwise (grid 0) by how much the second block of a compute unit has to do, one item
+// alone being quicker in the one-block form (attention alone, one MI355X, 256 compute units):
+//   dense D = 256, window items 144 / 252: 157 / 270 us one-block, 183 / 295 two-block;
+//         316 / 376 / 628 / 1024: 400 / 435 / 760 / 1302 and 322 / 366 / 662 / 1098;
+//   dense D = 128 (the one-block form's registers let two blocks share a unit there as
+//         well), 68 / 376 / 628: 230 / 205 / 380 and 326 / 245 / 417; 1024 / 2048: 722 / 1028
+//         and 674 / 1056;
+//   sparse D = 256: two-block 68-89 us against 77-104 at 20-72 window items, 298 / 558 against
+//         389 / 737 at 216 / 926, and up to 5 % behind where one long cluster ends the launch
+//         (136 items: 533 and 505);
+//   sparse D = 128: 252 us against 194 at 12 window items of 128 queries, 722 against 708 at 316.
+// A window's rows whose output offsets pass 31 bits go to the one-block form too.
 template <int D, int G>
 int launch_attn(const AttnArgs& a, int grid, hipStream_t stream) {
   static int pair_grid = 0, items_grid = 0;
   const int64_t window_out = ((int64_t)(PREFILL_ROWS / G - 1) * a.lo_sq + (int64_t)(G - 1) * a.lo_sh + D) * 2;
   const bool offsets_fit = window_out < INT32_MAX && (int64_t)a.Qc * a.Hq * 4 < INT32_MAX;
-  if (grid >= 0 && offsets_fit) return launch_attn_kernel<D>(attn_pair_kernel<D, G>, pair_grid, a, grid, stream);
+  const int64_t tiles = (a.Qc + PREFILL_ROWS / G - 1) / (PREFILL_ROWS / G) * (int64_t)a.Hkv;
+  const int64_t pair_from = a.nvis ? (D == 256 ? 0 : 33) : (D == 256 ? 257 : 769);
+  const bool pair = grid > 0 || (grid == 0 && tiles >= pair_from);
+  if (pair && offsets_fit) return launch_attn_kernel<D>(attn_pair_kernel<D, G>, pair_grid, a, grid, stream);
   return launch_attn_kernel<D>(attn_items_kernel<D, G>, items_grid, a, grid, stream);
 }
 

@@ -67,15 +67,14 @@ def fused_decode_step(layer, arena, *, q_post: torch.Tensor, q_pre: torch.Tensor
     qp = q_pre.reshape(hq, d)
     if q.stride(-1) != 1 or qp.stride(-1) != 1:
         raise ValueError("q_post and q_pre need unit inner strides")
-    pos = positions[:1]
-    if pos.dtype != torch.int32:
+    if positions.shape[0] < 1 or positions.dtype != torch.int32:
         raise ValueError("positions must be int32 (converting would allocate inside a capture)")
     kk = vv = kp = None
     if k_post is not None and v_states is not None:
         kk = k_post.reshape(hkv, d)
         vv = v_states.reshape(hkv, d)
         # the step reads both with K's row stride
-        if (hkv > 1 and vv.stride(0) != kk.stride(0)) or kk.stride(-1) != 1 or vv.stride(-1) != 1:
+        if kk.stride() != vv.stride() and hkv > 1 or kk.stride(1) != 1 or vv.stride(1) != 1:
             raise ValueError("k_post and v_states need unit inner strides and one row stride")
         if k_pre is not None and getattr(arena, "suffix_kpre", None) is not None:
             kp = k_pre.reshape(hkv, d)
@@ -83,7 +82,7 @@ def fused_decode_step(layer, arena, *, q_post: torch.Tensor, q_pre: torch.Tensor
                 raise ValueError("k_pre must share k_post's row layout (the step stores both)")
     out = output.reshape(hq, d)
     head = (_lib.ptr(q), q.stride(0), _lib.ptr(qp), qp.stride(0), 1,
-            _lib.ptr(kk), _lib.ptr(vv), kk.stride(0) if kk is not None else 0, _lib.ptr(pos),
+            _lib.ptr(kk), _lib.ptr(vv), kk.stride(0) if kk is not None else 0, _lib.ptr(positions),
             _lib.ptr(arena.codebooks), _lib.ptr(arena.sizes), _lib.ptr(arena.indptr),
             _lib.ptr(arena.packed_kv), arena.packed_kv.shape[1], _lib.ptr(arena.suffix_kv),
             arena.suffix_kv.shape[1], arena.suffix_block, _lib.ptr(arena.suffix_table),
