@@ -1330,10 +1330,12 @@ int launch_attn_kernel(AttnKernel kernel, int& auto_grid, const AttnArgs& a, int
 //   dense D = 128 (the one-block form's registers let two blocks share a unit there as
 //         well), 68 / 376 / 628: 230 / 205 / 380 and 326 / 245 / 417; 1024 / 2048: 722 / 1028
 //         and 674 / 1056;
-//   sparse D = 256: two-block 68-89 us against 77-104 at 20-72 window items, 298 / 558 against
-//         389 / 737 at 216 / 926, and up to 5 % behind where one long cluster ends the launch
-//         (136 items: 533 and 505);
-//   sparse D = 128: 252 us against 194 at 12 window items of 128 queries, 722 against 708 at 316.
+//   sparse, by the chunk's window items and the clusters' mean length up to the window
+//         (with few queries a launch ends with its longest cluster items, alone on their
+//         units): D = 256, length 40-220: two-block 68-89 us against 77-104 at 20-72 items,
+//         298 / 558 against 389 / 737 at 216 / 926; length 315 / 786: 432 / 533 against
+//         416 / 505 at 236 / 136; D = 128: 252 against 194 at 12 items, 722 against 708 at
+//         316, two-block from there (264 against 312 at 376 with the earlier one-block form).
 // A window's rows whose output offsets pass 31 bits go to the one-block form too.
 template <int D, int G>
 int launch_attn(const AttnArgs& a, int grid, hipStream_t stream) {
@@ -1341,7 +1343,8 @@ int launch_attn(const AttnArgs& a, int grid, hipStream_t stream) {
   const int64_t window_out = ((int64_t)(PREFILL_ROWS / G - 1) * a.lo_sq + (int64_t)(G - 1) * a.lo_sh + D) * 2;
   const bool offsets_fit = window_out < INT32_MAX && (int64_t)a.Qc * a.Hq * 4 < INT32_MAX;
   const int64_t tiles = (a.Qc + PREFILL_ROWS / G - 1) / (PREFILL_ROWS / G) * (int64_t)a.Hkv;
-  const int64_t pair_from = a.nvis ? (D == 256 ? 0 : 33) : (D == 256 ? 257 : 769);
+  const bool long_runs = D == 128 || a.wstart > (int64_t)a.C * 256;
+  const int64_t pair_from = a.nvis ? (long_runs ? 257 : 0) : (D == 256 ? 257 : 769);
   const bool pair = grid > 0 || (grid == 0 && tiles >= pair_from);
   if (pair && offsets_fit) return launch_attn_kernel<D>(attn_pair_kernel<D, G>, pair_grid, a, grid, stream);
   return launch_attn_kernel<D>(attn_items_kernel<D, G>, items_grid, a, grid, stream);

@@ -689,19 +689,22 @@ __global__ __launch_bounds__(1024) void build_items_kernel(const int32_t* __rest
     }
     __syncthreads();
   }
-  // expansion: a thread per window tile, then a wave per cluster source (its
-  // lanes write the items side by side)
+  // expansion: a thread per window tile, then a wave per cluster source (its lanes
+  // write the items side by side), or eight lanes where a cluster has few items (494
+  // queries of 16 heads on 4: the kernel takes 24 us with a wave each, 10 with a
+  // thread each, which at 8192 queries takes twice the wave form's 43)
   for (int s = threadIdx.x; s < nloc * hkv; s += 1024) {
     const ItemSource si = item_source(rev_counts, s_order, s, nloc, hkv, C, Qc, QT);
     if (s_first[s] < cap) items[s_first[s]] = PrefillItem{si.h, si.c, si.qb, si.qn, 0, 0, 0, 0};
   }
-  for (int s = nloc * hkv + wave; s < nsrc; s += 16) {
+  const int gl = (Qc + QT - 1) / QT > 64 ? 64 : 8, sub = threadIdx.x & (gl - 1);
+  for (int s = nloc * hkv + threadIdx.x / gl; s < nsrc; s += 1024 / gl) {
     const ItemSource si = item_source(rev_counts, s_order, s, nloc, hkv, C, Qc, QT);
     if (!si.n) continue;
     const int64_t f0 = s_first[s];
     const int e = si.h * C + si.c;
     const int nk = nvis[e], ent = rev_indptr[e], row = indptr[si.h * (C + 1) + si.c];
-    for (int j = lane; j < si.n; j += 64)
+    for (int j = sub; j < si.n; j += gl)
       if (f0 + j < cap) items[f0 + j] = PrefillItem{si.h, si.c, j * QT, min(QT, si.qn - j * QT), nk, ent + j * QT, row, 0};
   }
 }

@@ -90,7 +90,7 @@ def test_sparse_chunk_matches_fp64_over_the_selected_set(cfg):
 
 @pytest.mark.parametrize("cfg", [dict(hq=16, hkv=4, d=256, grid=8), dict(hq=8, hkv=2, d=128, grid=0)])
 def test_sparse_chunk_redone_when_keys_tower_over_the_first_tile(cfg):
-    """Sparse chunk (the pipelined kernel form): the index is built on ordinary keys,
+    """Sparse chunk (the two-block kernel form on a grid of 8): the index is built on ordinary keys,
     the attention reads keys of which every 97th lies far along the queries' common
     direction, so items whose cluster run (or window) holds one past its first tile
     pass 2^64 and are redone with the rows' true maxima.  On a grid of 8 blocks each
