@@ -426,9 +426,10 @@ class TokenOuterPrefillSession:
         if self._spare is None:
             self._spare = torch.zeros_like(packed)
         dst = self._spare
+        # the copy's rows lie n_so_far apart (a single row's stride() may still say otherwise)
         old_rows = index._inverse_positions[:, :n_so_far].clone()
         _lib.call("sbsa_repack_runs", _lib.ptr(packed), _lib.ptr(dst), width, hkv, d, n_so_far,
-                  _lib.ptr(old_rows), old_rows.stride(0), _lib.ptr(index.bucket_indptr), _lib.ptr(new_ip),
+                  _lib.ptr(old_rows), n_so_far, _lib.ptr(index.bucket_indptr), _lib.ptr(new_ip),
                   c, _lib.ptr(index.posting_positions), index.posting_positions.shape[1],
                   _lib.ptr(index._inverse_positions), index._inverse_positions.shape[1],
                   _lib.stream(packed.device))
