@@ -222,9 +222,12 @@ int sbsa_prefill_item_rows(void);
  * attention writes nothing and sbsa_prefill_combine (given the flag) skips the
  * chunk, which the caller runs again with a partial buffer of its exact size
  * (the reference reads the count instead, kv_outer.py:592-613).
- * queries_per_item = 128 / (Hq/Hkv). */
+ * queries_per_item = 128 / (Hq/Hkv).  The list's builder holds its sources in
+ * LDS: more than sbsa_prefill_items_max_queries queries with a window are refused
+ * (SBSA_ERR_UNSUPPORTED). */
 int64_t sbsa_prefill_items_bound(int64_t nnz, int num_queries, int num_kv_heads,
                                  int num_clusters, int queries_per_item);
+int64_t sbsa_prefill_items_max_queries(int num_kv_heads, int num_clusters, int queries_per_item);
 int sbsa_prefill_items(const int32_t* rev_counts, int num_kv_heads, int num_clusters,
                        int num_queries, int queries_per_item, int has_local,
                        const int32_t* indptr, const int32_t* nvis, const int32_t* rev_indptr,

@@ -736,14 +736,17 @@ void launch_reverse_index(const int32_t* qmask, int num_queries, int hkv, int C,
                      rev_counts, rev_indptr, qvals, qrank);
 }
 
+// The builder keeps each source's first item, and the cluster sources' keys and order, in LDS.
+constexpr int64_t ITEMS_LDS_BYTES = 150 * 1024;
+
 int launch_items(const int32_t* rev_counts, int hkv, int C, int num_queries, int queries_per_item, int has_local,
                  const int32_t* indptr, const int32_t* nvis, const int32_t* rev_indptr, void* items,
                  int64_t items_cap, int64_t partials_cap, int64_t last_partials_cap, int32_t* queue, int chunks,
                  const ChunkBatch& cb, hipStream_t stream) {
   const int nloc = has_local ? (num_queries + queries_per_item - 1) / queries_per_item : 0;
-  const size_t lds = (size_t)(nloc * hkv + 3 * hkv * C) * 4;
-  if (lds > 150 * 1024) return SBSA_ERR_UNSUPPORTED;
-  static size_t configured = 0;
+  const int64_t lds = ((int64_t)nloc * hkv + 3 * (int64_t)hkv * C) * 4;
+  if (lds > ITEMS_LDS_BYTES) return SBSA_ERR_UNSUPPORTED;
+  static int64_t configured = 0;
   if (lds > configured) {
     if (hipFuncSetAttribute((const void*)build_items_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
                             (int)lds) != hipSuccess)
@@ -883,6 +886,12 @@ int64_t sbsa_prefill_items_bound(int64_t nnz, int num_queries, int num_kv_heads,
   int64_t qt = queries_per_item;
   return (int64_t)num_kv_heads * ((num_queries + qt - 1) / qt) +
          (int64_t)num_kv_heads * num_clusters + (nnz + qt - 1) / qt;
+}
+
+int64_t sbsa_prefill_items_max_queries(int num_kv_heads, int num_clusters, int queries_per_item) {
+  if (num_kv_heads < 1 || num_clusters < 1 || queries_per_item < 1) return 0;
+  const int64_t tiles = (ITEMS_LDS_BYTES / 4 - 3 * (int64_t)num_kv_heads * num_clusters) / num_kv_heads;
+  return tiles > 0 ? tiles * queries_per_item : 0;
 }
 
 int sbsa_prefill_items(const int32_t* rev_counts, int num_kv_heads, int num_clusters,

@@ -46,6 +46,7 @@ SIGNATURES = {
     "sbsa_reverse_index_ints": (I64, [I32, I32, I32]),
     "sbsa_reverse_index": (I32, [P, I32, I32, I32, P, P, P, P, P, I64, P, P]),
     "sbsa_prefill_items_bound": (I64, [I64, I32, I32, I32, I32]),
+    "sbsa_prefill_items_max_queries": (I64, [I32, I32, I32]),
     "sbsa_prefill_items": (I32, [P, I32, I32, I32, I32, I32, P, P, P, P, I64, I64, P, P]),
     "sbsa_plan_chunks": (I32, [P, I64, I64, P, P, I64, P, P, I64, I32, I32, I32, I32, I32, I32, F32, F32, F32, I32,
                                I32, P, P, P, P, P, P, P, P, P, P, I64, I64, I64, P, P]),

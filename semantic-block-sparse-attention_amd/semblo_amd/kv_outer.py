@@ -380,6 +380,15 @@ def _zero_counts(n: int, dev) -> torch.Tensor:
     return z
 
 
+# clusters in the (empty) counts of a dense chunk's work list
+DENSE_CLUSTERS = 32
+
+
+def dense_launch_queries(num_kv_heads: int, q_per_kv: int) -> int:
+    """The most queries ``dense_causal_attention`` takes in one call."""
+    return _lib.query("sbsa_prefill_items_max_queries", num_kv_heads, DENSE_CLUSTERS, queries_per_item(q_per_kv))
+
+
 def dense_causal_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *, sm_scale: float,
                            chunk_start: int = 0, out: torch.Tensor | None = None,
                            grid: int | None = None, timing=None) -> torch.Tensor:
@@ -395,7 +404,7 @@ def dense_causal_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *,
     if k.shape[0] < chunk_start + qn:
         raise ValueError("k/v must cover every position up to the chunk's last query")
     qt = queries_per_item(g)
-    zero_counts = _zero_counts(hkv * 32, dev)
+    zero_counts = _zero_counts(hkv * DENSE_CLUSTERS, dev)
     bound = hkv * ((qn + qt - 1) // qt) + 1
     items = torch.empty(bound, ITEM_INTS, dtype=torch.int32, device=dev)
     queue = torch.empty(QUEUE_INTS, dtype=torch.int32, device=dev)
@@ -403,12 +412,12 @@ def dense_causal_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *,
         out = torch.empty_like(q)
     s = _lib.stream(dev)
     # no cluster has queries: the index arrays are never read
-    _lib.call("sbsa_prefill_items", _lib.ptr(zero_counts), hkv, 32, qn, qt, 1, _lib.ptr(zero_counts),
+    _lib.call("sbsa_prefill_items", _lib.ptr(zero_counts), hkv, DENSE_CLUSTERS, qn, qt, 1, _lib.ptr(zero_counts),
               _lib.ptr(zero_counts), _lib.ptr(zero_counts), _lib.ptr(items), bound, 0, _lib.ptr(queue), s)
     if timing is not None:
         timing.begin(s, "dense")
     _lib.call("sbsa_prefill_attend", _lib.ptr(q), q.stride(0), q.stride(1), qn, hq, hkv, d,
-              None, 0, _lib.ptr(k), _lib.ptr(v), k.stride(0), k.stride(1), None, None, 32, None,
+              None, 0, _lib.ptr(k), _lib.ptr(v), k.stride(0), k.stride(1), None, None, DENSE_CLUSTERS, None,
               None, _lib.ptr(items), _lib.ptr(queue), None, None,
               _lib.ptr(out), out.stride(0), out.stride(1), None, int(chunk_start), 0,
               float(sm_scale), int(grid or 0), s)

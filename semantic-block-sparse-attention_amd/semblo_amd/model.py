@@ -33,15 +33,21 @@ from .config import SembloRuntimeConfig, fitted_sink_tokens
 from .fused_decode import fused_decode_step
 from .fused_prefill import (PLAN_GROUP_QUERIES, CausalSnapshot, fused_chunk_execute, fused_chunk_plan,
                             fused_chunks_plan)
-from .kv_outer import PartialsGuard
-from .kv_outer import dense_causal_attention
+from .kv_outer import PartialsGuard, dense_causal_attention, dense_launch_queries
 from .state import ProductPostingIndex
 from .trivial_router import trivial_router_vectors
 
 
-# Most queries of one dense launch beside the index build: the work list of 65536 queries fits the
-# 150 KB its builder takes for up to 8 KV heads.
+# Most queries of one dense launch beside the index build (fewer where the work list takes fewer)
 DENSE_LAUNCH_QUERIES = 65536
+
+
+def dense_spans(queries: int, step: int, num_kv_heads: int, q_per_kv: int) -> list[tuple[int, int]]:
+    """The dense-prefix launches of a layer-major prefill: as many whole chunks of ``step``
+    queries to one as a launch takes."""
+    most = min(DENSE_LAUNCH_QUERIES, dense_launch_queries(num_kv_heads, q_per_kv))
+    per_launch = max(1, most // step) * step
+    return [(start, min(queries, start + per_launch)) for start in range(0, queries, per_launch)]
 
 
 _BUILD_STREAMS = threading.local()
@@ -314,9 +320,7 @@ class SembloAttention:
         # row), and the launch's items, longest first, fill its tail.  grid -1: with room for
         # the build's kernels on every compute unit.
         dense_end = min(length, -(-min(length, cap + 1) // step) * step)
-        per_launch = max(1, DENSE_LAUNCH_QUERIES // step) * step
-        for start in range(0, dense_end, per_launch):
-            end = min(dense_end, start + per_launch)
+        for start, end in dense_spans(dense_end, step, self.num_kv_heads, self.num_heads // self.num_kv_heads):
             if timing is not None:
                 n = end - start
                 timing.add_flops(4.0 * self.head_dim * self.num_heads * (n * (start + 1) + n * (n - 1) // 2))

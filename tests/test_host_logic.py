@@ -187,3 +187,23 @@ def test_flush_range_keeps_the_newest_and_moves_the_rest():
     assert all(b - a == every for a, b in moved)
     assert flush_range(length, 10 ** 6, length, keep, 0) is None          # flush off
     assert flush_layer(object(), 1200, 1200) == 0                         # nothing to move
+
+
+@pytest.mark.parametrize("hkv,g", [(1, 8), (4, 4), (8, 8), (10, 8), (16, 8), (16, 1), (32, 4), (64, 1), (64, 8)])
+@pytest.mark.parametrize("queries,step", [(1, 8192), (40960, 8192), (131072, 8192), (70001, 1000), (300000, 65536)])
+def test_dense_launches_fit_the_work_list(hkv, g, queries, step):
+    """A layer-major prefill puts several dense chunks into one launch; each launch's work list
+    (4 bytes per window tile and 12 per (head, cluster) of an empty list of 32) must fit the
+    150 KB its builder takes, and a launch is never less than one chunk."""
+    from semblo_amd import _lib, model
+    if not _lib.LIB_PATH.exists():
+        pytest.skip("libsbsa.so is not built here")
+    qt = 128 // g
+    spans = model.dense_spans(queries, step, hkv, g)
+    assert [a for a, _ in spans] + [queries] == [0] + [b for _, b in spans]
+    for a, b in spans:
+        fits = (-(-(b - a) // qt) * hkv + 3 * hkv * 32) * 4 <= 150 * 1024
+        assert fits or b - a <= step
+        assert a % step == 0 and b - a <= max(step, 65536)
+    most = _lib.query("sbsa_prefill_items_max_queries", hkv, 32, qt)
+    assert (-(-most // qt) * hkv + 96 * hkv) * 4 <= 150 * 1024 < ((-(-most // qt) + 1) * hkv + 96 * hkv) * 4
