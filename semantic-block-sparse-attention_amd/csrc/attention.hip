@@ -732,7 +732,7 @@ __global__ __launch_bounds__(256, 1) void attn_items_kernel(AttnArgs a) {
 // dense chunk of 8192 queries at 24576, 3564 -> 2967 us (1080 -> 1297 TFLOP/s;
 // an 8192^3 bf16 matrix product reaches 1313 there); a sparse chunk of 8192 at
 // 114688 (980K entries), 2328 -> 1846 us (750 -> 946 TFLOP/s); D = 128, a sparse
-// chunk of 3001 at 40009, 312 -> 252 us.
+// chunk of 3001 at 40009 with 16 heads on 8, 396 -> 348 us.
 template <int D, int G>
 __global__ __launch_bounds__(256, 2) void attn_pair_kernel(AttnArgs a) {
   using S = AttnTileShape<D>;
@@ -1300,6 +1300,17 @@ __global__ __launch_bounds__(256) void combine_kernel(
   if (out_lse && (lane * E) % D == 0) out_lse[(int64_t)qi * Hq + h * G + j] = mx + logf(den);
 }
 
+int compute_units() {
+  static int units = 0;
+  if (!units) {
+    int dev = 0, cus = 0;
+    (void)hipGetDevice(&dev);
+    (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
+    units = cus > 0 ? cus : 256;
+  }
+  return units;
+}
+
 // Launches one of the two forms with a grid that fills the GPU (or the caller's).
 using AttnKernel = void (*)(AttnArgs);
 template <int D>
@@ -1308,11 +1319,9 @@ int launch_attn_kernel(AttnKernel kernel, int& auto_grid, const AttnArgs& a, int
   if (!auto_grid) {
     if (hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
       return SBSA_ERR_UNSUPPORTED;
-    int dev = 0, cus = 0, occ = 0;
-    (void)hipGetDevice(&dev);
-    (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
+    int occ = 0;
     (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, (const void*)kernel, 256, lds);
-    auto_grid = (cus > 0 ? cus : 256) * (occ > 0 ? occ : 1);
+    auto_grid = compute_units() * (occ > 0 ? occ : 1);
   }
   hipLaunchKernelGGL(kernel, dim3(grid > 0 ? grid : auto_grid), dim3(256), lds, stream, a);
   return SBSA_OK;
@@ -1324,18 +1333,24 @@ int launch_attn_kernel(AttnKernel kernel, int& auto_grid, const AttnArgs& a, int
 // register, so the build would follow it: prefill of 32768 5.5 ms with the one-block dense
 // chunks, 6.8 with these; of 131072 42.1 and 42.7).  An explicit grid gets the two-block form.
 // Otherwise (grid 0) by how much the second block of a compute unit has to do, one item
-// alone being quicker in the one-block form (attention alone, one MI355X, 256 compute units):
-//   dense D = 256, window items 144 / 252: 157 / 270 us one-block, 183 / 295 two-block;
-//         316 / 376 / 628 / 1024: 400 / 435 / 760 / 1302 and 322 / 366 / 662 / 1098;
-//   dense D = 128 (the one-block form's registers let two blocks share a unit there as
-//         well), 68 / 376 / 628: 230 / 205 / 380 and 326 / 245 / 417; 1024 / 2048: 722 / 1028
-//         and 674 / 1056;
-//   sparse, by the chunk's window items and the clusters' mean length up to the window
-//         (with few queries a launch ends with its longest cluster items, alone on their
-//         units): D = 256, length 40-220: two-block 68-89 us against 77-104 at 20-72 items,
-//         298 / 558 against 389 / 737 at 216 / 926; length 315 / 786: 432 / 533 against
-//         416 / 505 at 236 / 136; D = 128: 252 against 194 at 12 items, 722 against 708 at
-//         316, two-block from there (264 against 312 at 376 with the earlier one-block form).
+// alone being quicker in the one-block form.  Attention alone, one MI355X, one-block against
+// two-block us, by the chunk's window items (T) and the 256 compute units (U):
+//   D = 128 with 4 or 8 heads per KV head: two blocks of the one-block form share a unit (its
+//     253 registers; 258 and 264 with 1 and 2 heads), and it is the quicker at every size:
+//     dense T 88 / 512 / 1024: 177 / 355 / 1455 and 244 / 383 / 1505, sparse, 46 chunks of
+//     200 to 8192 queries: 0.67 to 1.01 of the two-block form's time.
+//   D = 128 with 1 or 2 heads: two-block from T = 5/4 U.  Dense T 256 / 320 / 376 / 512 / 1024:
+//     512 / 358 / 347 / 866 / 1734 and 727 / 358 / 313 / 798 / 1446; sparse T 256: 211-712 and
+//     260-960 (one chunk of three 447 and 390), T 376 / 512 / 1024: 391 / 435 / 1654 and
+//     348 / 372 / 1194.
+//   D = 256 dense: two-block once a unit has a second item.  T 188 / 256 / 264 / 1024: 313 / 344 /
+//     531 / 2972 and 362 / 385 / 388 / 2569.
+//   D = 256 sparse: with few queries a launch ends with its longest cluster items, alone on
+//     their units, so the clusters' mean length up to the window counts as well.  111 chunks of
+//     200 to 8192 queries, 8K to 390K positions: with 4 or 8 heads per KV head (more items of a
+//     cluster for the same queries) two-block from T = U/2 or up to a length of 256, mean 1.02 of
+//     the better form's time (from T = U + 1: 1.06; one-block always: 1.11); with 1 or 2 heads
+//     from T = U + 1, 1.01 (as for 4 and 8 heads 1.04).
 // A window's rows whose output offsets pass 31 bits go to the one-block form too.
 template <int D, int G>
 int launch_attn(const AttnArgs& a, int grid, hipStream_t stream) {
@@ -1343,9 +1358,11 @@ int launch_attn(const AttnArgs& a, int grid, hipStream_t stream) {
   const int64_t window_out = ((int64_t)(PREFILL_ROWS / G - 1) * a.lo_sq + (int64_t)(G - 1) * a.lo_sh + D) * 2;
   const bool offsets_fit = window_out < INT32_MAX && (int64_t)a.Qc * a.Hq * 4 < INT32_MAX;
   const int64_t tiles = (a.Qc + PREFILL_ROWS / G - 1) / (PREFILL_ROWS / G) * (int64_t)a.Hkv;
-  const bool long_runs = D == 128 || a.wstart > (int64_t)a.C * 256;
-  const int64_t pair_from = a.nvis ? (long_runs ? 257 : 0) : (D == 256 ? 257 : 769);
-  const bool pair = grid > 0 || (grid == 0 && tiles >= pair_from);
+  const int64_t units = compute_units();
+  bool two_blocks = tiles > units;
+  if (D == 128) two_blocks = G <= 2 && 4 * tiles >= 5 * units;
+  if (D == 256 && G >= 4 && a.nvis) two_blocks = 2 * tiles >= units || a.wstart <= (int64_t)a.C * 256;
+  const bool pair = grid > 0 || (grid == 0 && two_blocks);
   if (pair && offsets_fit) return launch_attn_kernel<D>(attn_pair_kernel<D, G>, pair_grid, a, grid, stream);
   return launch_attn_kernel<D>(attn_items_kernel<D, G>, items_grid, a, grid, stream);
 }
