@@ -1348,9 +1348,10 @@ int launch_attn_kernel(AttnKernel kernel, int& auto_grid, const AttnArgs& a, int
 //   D = 256 sparse: with few queries a launch ends with its longest cluster items, alone on
 //     their units, so the clusters' mean length up to the window counts as well.  111 chunks of
 //     200 to 8192 queries, 8K to 390K positions: with 4 or 8 heads per KV head (more items of a
-//     cluster for the same queries) two-block from T = U/2 or up to a length of 256, mean 1.02 of
-//     the better form's time (from T = U + 1: 1.06; one-block always: 1.11); with 1 or 2 heads
-//     from T = U + 1, 1.01 (as for 4 and 8 heads 1.04).
+//     cluster for the same queries) two-block from T = U + 1 or up to a length of 256, mean 1.04 of
+//     the better form's time (by T alone 1.06; one-block always 1.11; from T = U/2 1.02, but
+//     single chunks then lose much: 1115 queries at 90000 453 -> 533 us); with 1 or 2 heads by T
+//     alone, 1.01 (with the length 1.05).
 // A window's rows whose output offsets pass 31 bits go to the one-block form too.
 template <int D, int G>
 int launch_attn(const AttnArgs& a, int grid, hipStream_t stream) {
@@ -1361,7 +1362,7 @@ int launch_attn(const AttnArgs& a, int grid, hipStream_t stream) {
   const int64_t units = compute_units();
   bool two_blocks = tiles > units;
   if (D == 128) two_blocks = G <= 2 && 4 * tiles >= 5 * units;
-  if (D == 256 && G >= 4 && a.nvis) two_blocks = 2 * tiles >= units || a.wstart <= (int64_t)a.C * 256;
+  if (D == 256 && G >= 4 && a.nvis) two_blocks = tiles > units || a.wstart <= (int64_t)a.C * 256;
   const bool pair = grid > 0 || (grid == 0 && two_blocks);
   if (pair && offsets_fit) return launch_attn_kernel<D>(attn_pair_kernel<D, G>, pair_grid, a, grid, stream);
   return launch_attn_kernel<D>(attn_items_kernel<D, G>, items_grid, a, grid, stream);

@@ -49,7 +49,7 @@ def test_dense_chunk_past_an_item_per_unit(hkv, g, d, share):
     (2, 8, 256, 0.1, 10000, None, False), (2, 8, 256, 0.1, 10000, None, True),      # one block: long runs
     (2, 8, 256, 0.1, 5000, -1, True), (4, 4, 256, 0.2, 10000, None, True),
     (2, 8, 256, 0.1, 5000, None, True),                                             # two: short runs
-    (2, 8, 256, 0.6, 10000, None, False), (4, 4, 256, 0.6, 10000, None, True),      # two: items
+    (4, 4, 256, 0.9, 10000, None, True), (2, 8, 256, 1.1, 10000, None, False),      # one, two: items
     (8, 2, 256, 0.9, 5000, None, False), (16, 2, 256, 1.1, 10000, None, False),     # one, two
     (16, 2, 128, 1.1, 5000, None, True), (16, 2, 128, 1.4, 5000, None, True),       # one, two
     (16, 1, 128, 1.4, 5000, None, False), (4, 8, 128, 1.4, 5000, None, True)])      # two, one
