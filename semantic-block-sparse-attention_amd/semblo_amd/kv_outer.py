@@ -116,12 +116,18 @@ def kv_outer_attention(q: torch.Tensor, packed_kv: torch.Tensor, qmask: torch.Te
     counted = torch.cuda.Event()
     counted.record(torch.cuda.current_stream(dev))
     capped = _CappedChunk()
+    how = dict(sm_scale=sm_scale, local_kv=local_kv, chunk_start=chunk_start, wstart=wstart, out=out,
+               want_stats=want_stats, grid=grid, timing=timing)
+    room = True
     try:
-        out, stats = kv_outer_execute(q, packed_kv, plan, None, bucket_indptr, sm_scale=sm_scale,
-                                      local_kv=local_kv, chunk_start=chunk_start, wstart=wstart, out=out,
-                                      want_stats=want_stats, grid=grid, timing=timing, guard=capped)
+        out, stats = kv_outer_execute(q, packed_kv, plan, None, bucket_indptr, guard=capped, **how)
+    except torch.OutOfMemoryError:      # raised before the attention is enqueued
+        room = False
     finally:
         counted.synchronize()           # `count` is the kernel's until then
+    if not room:
+        # no memory for the bound: the rows at the exact count
+        out, stats = kv_outer_execute(q, packed_kv, plan, int(count[0]), bucket_indptr, **how)
     stats["partials"] = int(count[0])
     if capped.rerun is not None and stats["partials"] > partials_room(qn, hkv, c, g, d, q.element_size())[0]:
         capped.rerun()

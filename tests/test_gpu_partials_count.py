@@ -44,3 +44,16 @@ def test_the_count_comes_without_a_copy(qn, hkv, g, d, c, own_stream, monkeypatc
             assert stats["partials"] == want
     stream.synchronize()
     assert copies == [] and torch.equal(out, ref)
+
+
+def test_rows_at_the_exact_count_where_the_bound_does_not_fit(limit_memory):
+    """The bound of 4096 queries and 512 (head, cluster) takes 2.2 GB of rows, a twentieth of them
+    selected 0.1 GB."""
+    from semblo_amd.kv_outer import kv_outer_attention
+    args, kw, want = _chunk(4096, 4, 4, 128, 128, 0.05)
+    ref = kv_outer_attention(*args, **kw)[0]
+    limit_memory(600 << 20)
+    with pytest.raises(torch.OutOfMemoryError):
+        torch.empty(2 << 30, dtype=torch.uint8, device=DEV)
+    out, stats = kv_outer_attention(*args, **kw)
+    assert stats["partials"] == want and torch.equal(out, ref)
