@@ -238,8 +238,11 @@ class ProductPostingIndex:
             raise ValueError("product_keys must be bfloat16")
 
         if fit_trace is None and not sink:
-            fitted = _fit_batched(pk, seed=int(codebook_seed or 0), fit_n=fit_n, c=c, iters=iters,
-                                  align=max(align, 1), router_pass=bool(router_pass))
+            try:
+                fitted = _fit_batched(pk, seed=int(codebook_seed or 0), fit_n=fit_n, c=c, iters=iters,
+                                      align=max(align, 1), router_pass=bool(router_pass))
+            except torch.OutOfMemoryError:      # every head's key space at once: one after another
+                fitted = None
             if fitted is not None:
                 sizes, indptr, posting_full, inverse, codebooks, width = fitted
                 return cls(codebooks=codebooks, posting_positions=posting_full[:, :width].contiguous(),
