@@ -350,13 +350,17 @@ class SembloAttention:
             for i in range(0, len(sparse), per_call):
                 group = sparse[i:i + per_call]
                 first, last = group[0][0], group[-1][1]
-                with torch.cuda.stream(side):
-                    pls = fused_chunks_plan(qp[first:last], index, first, step,
-                                            temperature=cfg.selection_temperature, beta=cfg.bucket_size_penalty,
-                                            target_tokens=self.target_tokens, iters=cfg.iters, guard=guard,
-                                            keep_theta=self.plan_log is not None)
-                    ev = torch.cuda.Event()
-                    ev.record(side)
+                try:
+                    with torch.cuda.stream(side):
+                        pls = fused_chunks_plan(qp[first:last], index, first, step,
+                                                temperature=cfg.selection_temperature, beta=cfg.bucket_size_penalty,
+                                                target_tokens=self.target_tokens, iters=cfg.iters, guard=guard,
+                                                keep_theta=self.plan_log is not None)
+                        ev = torch.cuda.Event()
+                        ev.record(side)
+                except torch.OutOfMemoryError:      # the group's routing vectors: a chunk at a time
+                    self._plan_each(group, q, qp, index, side, guard, plans, ready)
+                    continue
                 for pl in pls:
                     pl.record(self.plan_log)
                 plans += pls
@@ -388,7 +392,7 @@ class SembloAttention:
 
     def _plan_each(self, sparse, q, qp, index, side, guard, plans, ready) -> None:
         """The chunks' plans one by one (with an attention sink, which the plans of several
-        chunks in one call do not take)."""
+        chunks in one call do not take, or where their memory is not there)."""
         cfg = self.runtime_config
         snapshot = CausalSnapshot(index)
         for st, en in sparse:
