@@ -37,11 +37,27 @@ def queries_per_item(q_per_kv: int) -> int:
     return _lib.query("sbsa_prefill_item_rows") // q_per_kv
 
 
-# From this many (query, KV head, cluster) on, a reverse index is given room for the counts
-# of query segments; fewer queries make too few segments (the two passes and the scan at
-# 512 (head, cluster): 13 us without and 25 with at 494 queries, even at about 3072, 55 and
-# 33 at 8192).
-SEGMENTS_FROM = 3072 * 512
+def segments_pay(num_queries: int, num_kv_heads: int, num_clusters: int) -> bool:
+    """Whether a reverse index is quicker in query segments, and is given room for their counts.
+
+    The form without room runs a block per (head, cluster), each over every query; the
+    segments run a block per 256 queries and head, each over every cluster of the head, and
+    one block that scans the segments' counts.  So the first grows with the queries, and with
+    (head, cluster) past two blocks per compute unit, the second with a head's clusters.  Us
+    without and with room, one MI355X (256 compute units), a fifth of the clusters selected:
+      heads x clusters   500 queries   2000     4096      8192
+      1 x 128            12 / 25       15 / 26  23 / 26   39 / 28
+      4 x 128            12 / 26       18 / 27  30 / 28   52 / 31
+      16 x 128           17 / 29       39 / 31  69 / 33   129 / 48
+      1 x 256            12 / 42       16 / 44  26 / 45   47 / 47
+      4 x 256            13 / 45       23 / 47  40 / 48   66 / 50
+      4 x 512            17 / 84       39 / 86  69 / 88   129 / 93
+      4 x 1024           27 / 160      74 / 168 134 / 172 266 / 179
+      1 x 1024           13 / 151      23 / 160 38 / 157  66 / 160
+    The line is where 8 + Q (4 + max(0, heads x clusters - 512) / 150) / 1000 us meets
+    6 + 0.155 clusters."""
+    lists = num_kv_heads * num_clusters
+    return num_queries * (4 + max(0, lists - 512) / 150) > 155 * num_clusters - 2000
 
 
 def build_reverse_index(qmask: torch.Tensor, live: torch.Tensor, *, num_queries: int,
@@ -62,7 +78,8 @@ def build_reverse_index(qmask: torch.Tensor, live: torch.Tensor, *, num_queries:
     nnz = torch.empty(1, dtype=torch.int64, device=dev) if count is None else count
     # the lists' bound, and room behind them for the kernels' counts
     bound = num_queries * hkv * c
-    cap = max(_lib.query("sbsa_reverse_index_ints", num_queries, hkv, c) if bound > SEGMENTS_FROM else bound, 1)
+    segments = segments_pay(num_queries, hkv, c)
+    cap = max(_lib.query("sbsa_reverse_index_ints", num_queries, hkv, c) if segments else bound, 1)
     qvals = torch.empty(cap, dtype=torch.int32, device=dev)
     qrank = torch.empty(num_queries, hkv, c, dtype=torch.int32, device=dev)
     live32 = live if live.dtype == torch.int32 and live.is_contiguous() else live.to(torch.int32).contiguous()

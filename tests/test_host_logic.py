@@ -207,3 +207,14 @@ def test_dense_launches_fit_the_work_list(hkv, g, queries, step):
         assert a % step == 0 and b - a <= max(step, 65536)
     most = _lib.query("sbsa_prefill_items_max_queries", hkv, 32, qt)
     assert (-(-most // qt) * hkv + 96 * hkv) * 4 <= 150 * 1024 < ((-(-most // qt) + 1) * hkv + 96 * hkv) * 4
+
+
+@pytest.mark.parametrize("hkv,c,queries,want", [
+    (4, 128, 494, False), (4, 128, 8192, True), (1, 128, 2000, False), (1, 128, 8192, True),
+    (16, 128, 900, False), (16, 128, 2000, True), (4, 1024, 400, False), (4, 1024, 4096, False),
+    (4, 1024, 8192, True), (1, 1024, 16384, False), (4, 512, 4096, False), (4, 512, 8192, True)])
+def test_reverse_index_form_by_both_forms_blocks(hkv, c, queries, want):
+    """The reverse index's form follows what each form's blocks have to do (measured on either
+    side of each line), not the product of queries, heads and clusters."""
+    from semblo_amd.kv_outer import segments_pay
+    assert segments_pay(queries, hkv, c) is want
