@@ -51,6 +51,7 @@ def dense_spans(queries: int, step: int, num_kv_heads: int, q_per_kv: int) -> li
 
 
 _BUILD_STREAMS = threading.local()
+BUILD_STREAMS_KEPT = 32         # torch's pool has this many streams
 
 
 class SembloQueryState:
@@ -165,15 +166,21 @@ class SembloAttention:
         index.original_kv = (k_post, v)
         return index
 
-    def _build_stream(self, device) -> torch.cuda.Stream:
-        """The stream the index is built on while the dense chunks run (default priority): one
-        per device and host thread, so that a new layer's build finds the memory that the
-        earlier layers' builds left to the stream (a stream of its own starts with none)."""
-        streams = _BUILD_STREAMS.__dict__.setdefault("by_device", {})
-        device = torch.device(device)
-        if device not in streams:
-            streams[device] = torch.cuda.Stream(device=device)
-        return streams[device]
+    def _build_stream(self, main: torch.cuda.Stream) -> torch.cuda.Stream:
+        """The stream the index is built on while the dense chunks run on ``main`` (default
+        priority): one per host thread and stream of the caller's, so that a new layer's build
+        finds the memory that the earlier layers' builds left to the stream (a stream of its own
+        starts with none), and layers run on different streams do not follow each other's builds."""
+        streams = _BUILD_STREAMS.__dict__.setdefault("by_main", {})
+        side = streams.get(main)
+        if side is None:
+            if len(streams) >= BUILD_STREAMS_KEPT:
+                streams.clear()
+            side = torch.cuda.Stream(device=main.device)
+            if side == main:            # the pool hands its streams out in turn
+                side = torch.cuda.Stream(device=main.device)
+            streams[main] = side
+        return side
 
     def begin_token_outer_prefill(self, tokens, chunk: int, **kw):
         """A token-order prefill session of a prompt (its length, or its positions as
@@ -326,7 +333,7 @@ class SembloAttention:
                 timing.add_flops(4.0 * self.head_dim * self.num_heads * (n * (start + 1) + n * (n - 1) // 2))
             dense_causal_attention(q[start:end], kk, vv, sm_scale=self.scaling, chunk_start=start,
                                    out=out[start:end], grid=-1, timing=timing)
-        side = self._build_stream(q.device)
+        side = self._build_stream(main)
         side.wait_event(inputs_ready)
         sparse = [(st, min(length, st + step)) for st in range(0, length, step) if st > cap]
         # every sparse chunk's plan (selection, reverse index, work list) on the build
