@@ -139,11 +139,19 @@ int sbsa_bucket_layout(const int32_t* assign, int64_t length, int num_clusters, 
  * [heads, 2, C, dim/2]; totals [heads + 1]: the padded totals, and the first head
  * that left clusters empty in more than `ahead` iterations (else `heads`): that
  * head and those after it are not valid.  dim in {64, 128, 256}, rows 16-byte
- * aligned, the workspace 256-byte aligned. */
+ * aligned, the workspace 256-byte aligned.
+ *
+ * To go on from a head that was not valid: sbsa_kmeans_fit_counted also writes
+ * restarts_made (one int on the device, or null), the restarts of the valid heads,
+ * and sbsa_kmeans_draws_after makes the draws that follow those of heads_before
+ * heads and restarts_before restarts.  One head alone is one fit, whatever it
+ * restarts, and valid with `ahead` = iters. */
 int64_t sbsa_kmeans_draw_ints(int64_t fit_n, int heads, int num_clusters, int ahead);
 int64_t sbsa_kmeans_draw_scratch_ints(int64_t length, int64_t fit_n, int heads, int ahead);
 int sbsa_kmeans_draws(uint32_t seed, int64_t length, int64_t fit_n, int heads, int num_clusters, int ahead,
                       int32_t* out, int32_t* scratch);
+int sbsa_kmeans_draws_after(uint32_t seed, int heads_before, int restarts_before, int64_t length, int64_t fit_n,
+                            int heads, int num_clusters, int ahead, int32_t* out, int32_t* scratch);
 size_t sbsa_kmeans_fit_workspace_bytes(int64_t length, int64_t fit_n, int heads, int num_clusters, int dim,
                                        int ahead, int iters);
 int sbsa_kmeans_fit(const void* keys, int64_t length, int64_t ld_k, int64_t ld_h, int heads, int dim,
@@ -151,6 +159,11 @@ int sbsa_kmeans_fit(const void* keys, int64_t length, int64_t ld_k, int64_t ld_h
                     int iters, int align, int32_t* sizes, int32_t* indptr, int32_t* posting,
                     int64_t posting_cap, int32_t* inverse, int32_t* totals, void* codebooks,
                     void* workspace, size_t workspace_bytes, hipStream_t stream);
+int sbsa_kmeans_fit_counted(const void* keys, int64_t length, int64_t ld_k, int64_t ld_h, int heads, int dim,
+                            int router_pass, const int32_t* draws, int64_t fit_n, int num_clusters, int ahead,
+                            int iters, int align, int32_t* sizes, int32_t* indptr, int32_t* posting,
+                            int64_t posting_cap, int32_t* inverse, int32_t* totals, int32_t* restarts_made,
+                            void* codebooks, void* workspace, size_t workspace_bytes, hipStream_t stream);
 
 /* ---- S1b: packed K/V --------------------------------------------------------
  * Replaces ProductPostingIndex.pack_prompt_kv (semblo/vllm_plugin/state.py:950-997):

@@ -634,19 +634,23 @@ __global__ void pack_kv_kernel(const bf16_t* __restrict__ key, const bf16_t* __r
 // before it (fit h + ahead h (h - 1) / 2 + r for r); flags[fit][iters] is the
 // number of iterations of that fit that left a cluster empty.  A head with more
 // than `ahead` of them needs restarts that were not drawn: *failed is the first
-// such head (else `heads`), and it and the later heads are not valid.
+// such head (else `heads`), and it and the later heads are not valid; *made is the
+// restarts that the valid heads made.
 __global__ void kmeans_resolve_kernel(const int32_t* __restrict__ flags, int iters, int heads, int ahead,
-                                      int32_t* __restrict__ pick, int32_t* __restrict__ failed) {
+                                      int32_t* __restrict__ pick, int32_t* __restrict__ failed,
+                                      int32_t* __restrict__ made) {
   if (threadIdx.x != 0) return;
-  int restarts = 0, bad = heads;
+  int restarts = 0, bad = heads, valid_restarts = 0;
   for (int h = 0; h < heads; ++h) {
     const int fit = h + ahead * (h * (h - 1) / 2) + (h < bad ? restarts : 0);
     pick[h] = fit;
     const int empties = flags[(int64_t)fit * (iters + 1) + iters];
     if (empties > ahead) bad = min(bad, h);
     restarts += empties;
+    if (h < bad) valid_restarts = restarts;
   }
   *failed = bad;
+  if (made) *made = valid_restarts;
 }
 
 // Vectorised forms of the two kernels above for rows of 64..512 elements with
@@ -1082,18 +1086,30 @@ static int64_t draw_words(int64_t length, int64_t fit_n, int heads, int ahead) {
 
 extern "C" int64_t sbsa_kmeans_draw_scratch_ints(int64_t length, int64_t fit_n, int heads, int ahead) {
   if (length < 1 || fit_n < 1 || heads < 1 || ahead < 1) return 0;
-  return draw_words(length, fit_n, heads, ahead) + length;
+  return draw_words(length, fit_n, heads, ahead) + 624 + length;     // 624: words before the first
 }
 
 extern "C" int sbsa_kmeans_draws(uint32_t seed, int64_t length, int64_t fit_n, int heads, int num_clusters, int ahead,
                                  int32_t* out, int32_t* scratch) {
-  if (!out || !scratch || !fit_shape_ok(length, fit_n, heads, num_clusters, 64, ahead, 1) || length >= (1ll << 27))
+  return sbsa_kmeans_draws_after(seed, 0, 0, length, fit_n, heads, num_clusters, ahead, out, scratch);
+}
+
+extern "C" int sbsa_kmeans_draws_after(uint32_t seed, int heads_before, int restarts_before, int64_t length,
+                                       int64_t fit_n, int heads, int num_clusters, int ahead, int32_t* out,
+                                       int32_t* scratch) {
+  if (!out || !scratch || !fit_shape_ok(length, fit_n, heads, num_clusters, 64, ahead, 1) || length >= (1ll << 27) ||
+      heads_before < 0 || restarts_before < 0)
     return SBSA_ERR_ARG;
   const int64_t head_words = (length - 1) + (fit_n - 1), n_words = draw_words(length, fit_n, heads, ahead);
   uint32_t* words = (uint32_t*)scratch;
   Mt19937 mt(seed);
-  for (int64_t i = 0; i < n_words; i += 624) mt.block(words + i);
-  int32_t* ident = scratch + n_words;
+  // the words of the draws before these: whole blocks are passed by, the rest lie before the first
+  const int64_t before = heads_before * head_words + restarts_before * (fit_n - 1);
+  for (int64_t i = 0; i < before / 624; ++i) mt.block(words);
+  const int64_t made = n_words + (before % 624 ? 624 : 0);
+  for (int64_t i = 0; i < made; i += 624) mt.block(words + i);
+  words += before % 624;
+  int32_t* ident = scratch + made;
   for (int64_t i = 0; i < length; ++i) ident[i] = (int32_t)i;
   const int64_t set = fit_n + (int64_t)(1 + ahead) * num_clusters;
   int32_t* head_of = out + num_fits(heads, ahead) * set;
@@ -1121,6 +1137,17 @@ extern "C" int sbsa_kmeans_fit(const void* keys, int64_t length, int64_t ld_k, i
                                int iters, int align, int32_t* sizes, int32_t* indptr, int32_t* posting,
                                int64_t posting_cap, int32_t* inverse, int32_t* totals, void* codebooks,
                                void* workspace, size_t workspace_bytes, hipStream_t stream) {
+  return sbsa_kmeans_fit_counted(keys, length, ld_k, ld_h, heads, dim, router_pass, draws, fit_n, num_clusters, ahead,
+                                 iters, align, sizes, indptr, posting, posting_cap, inverse, totals, nullptr,
+                                 codebooks, workspace, workspace_bytes, stream);
+}
+
+extern "C" int sbsa_kmeans_fit_counted(const void* keys, int64_t length, int64_t ld_k, int64_t ld_h, int heads,
+                                       int dim, int router_pass, const int32_t* draws, int64_t fit_n,
+                                       int num_clusters, int ahead, int iters, int align, int32_t* sizes,
+                                       int32_t* indptr, int32_t* posting, int64_t posting_cap, int32_t* inverse,
+                                       int32_t* totals, int32_t* restarts_made, void* codebooks, void* workspace,
+                                       size_t workspace_bytes, hipStream_t stream) {
   if (!keys || !draws || !sizes || !indptr || !posting || !inverse || !totals || !codebooks || !workspace)
     return SBSA_ERR_ARG;
   if (!fit_shape_ok(length, fit_n, heads, num_clusters, dim, ahead, iters) || align < 1) return SBSA_ERR_UNSUPPORTED;
@@ -1164,7 +1191,7 @@ extern "C" int sbsa_kmeans_fit(const void* keys, int64_t length, int64_t ld_k, i
                        (int64_t)dim, sample, num_clusters, dim, cent_f32, cent_bf16, flags + it, ahead, fb);
   }
   hipLaunchKernelGGL(kmeans_resolve_kernel, dim3(1), dim3(64), 0, stream, (const int32_t*)flags, iters, heads, ahead,
-                     pick, totals + heads);
+                     pick, totals + heads, restarts_made);
   FitBatch hb;              // per head, with the picked fits' centroids
   hb.pick = pick;
   hb.x = length * dim;

@@ -36,9 +36,12 @@ SIGNATURES = {
     "sbsa_kmeans_draw_ints": (I64, [I64, I32, I32, I32]),
     "sbsa_kmeans_draw_scratch_ints": (I64, [I64, I64, I32, I32]),
     "sbsa_kmeans_draws": (I32, [ctypes.c_uint32, I64, I64, I32, I32, I32, P, P]),
+    "sbsa_kmeans_draws_after": (I32, [ctypes.c_uint32, I32, I32, I64, I64, I32, I32, I32, P, P]),
     "sbsa_kmeans_fit_workspace_bytes": (SZ, [I64, I64, I32, I32, I32, I32, I32]),
     "sbsa_kmeans_fit": (I32, [P, I64, I64, I64, I32, I32, I32, P, I64, I32, I32, I32, I32, P, P, P, I64, P, P,
                               P, P, SZ, P]),
+    "sbsa_kmeans_fit_counted": (I32, [P, I64, I64, I64, I32, I32, I32, P, I64, I32, I32, I32, I32, P, P, P, I64, P,
+                                      P, P, P, P, SZ, P]),
     "sbsa_pack_kv": (I32, [P, P, I64, I64, I32, I32, P, I64, I64, P, P]),
     "sbsa_score_select": (I32, [P, I64, I64, P, P, P, I64, I64, I32, I32, I32, I32, I32, I32,
                                 F32, F32, F32, I32, I32, P, P, P, P, P, P, P]),

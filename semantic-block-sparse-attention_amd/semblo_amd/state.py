@@ -19,7 +19,7 @@ reference reads the cluster counts every k-means iteration (its
 ``empty.any()`` test).  Here every head's whole fit runs in one call, for
 every number of restarts the heads before it can have made, with one host
 read at the end (_fit_batched).  Where that call does not apply (a sink, a
-trace, large fits, a third empty iteration) the heads follow each other: the first RESTARTS_AHEAD restart draws of a head
+trace, large fits) the heads follow each other: the first RESTARTS_AHEAD restart draws of a head
 are made ahead and applied on the GPU at the first iterations that leave a
 cluster empty, the iterations run ahead, and one read of the counts tells
 how many draws were used: the generator's state is set back before the first
@@ -44,6 +44,8 @@ from .config import check_sink_partition, fitted_sink_tokens, num_flat_clusters
 PACK_ALIGN = 256
 # restart draws of the k-means fit made ahead per KV head (the GPU applies them)
 RESTARTS_AHEAD = 2
+# and at most, for a head fitted alone in one call
+RESTARTS_MOST = 8
 
 
 class _DrawBuffers:
@@ -84,10 +86,12 @@ def _draw_buffers(length: int, fit_n: int, c: int) -> _DrawBuffers:
 
 # The batched fit runs every head's fit for every number of restarts the heads before it
 # can have made (1 + RESTARTS_AHEAD h fits for head h).  That is worth it while a k-means
-# iteration is a chain of short launches: past BATCH_WORK (fits x sample rows x centroids)
-# the fits that are not used are expected to cost more than the host's waits between the
-# heads (the line itself is an estimate, not a measured crossing; below it, 4 KV heads of
-# D = 256, 32768 positions, 128 clusters, beside the dense chunks: 3.9 -> 2.0 ms).
+# iteration is a chain of short launches.  Every shape measured up to BATCH_WORK (fits x
+# sample rows x centroids: 8 KV heads, 64 fits, at 8192 rows and 128 clusters) builds faster
+# than head after head, alone on one MI355X: 1 / 2 / 4 / 8 heads of D = 256 at 8192 positions
+# 607 / 1125 / 2039 / 3957 -> 485 / 606 / 927 / 2507 us, at 131072 1343 / 2505 / 4672 / 9381
+# -> 603 / 817 / 1414 / 3833 (beside the dense chunks, 4 heads at 32768: 3.9 -> 2.0 ms).
+# Larger ones were not measured, and go head after head.
 BATCH_FITS = 64
 BATCH_WORK = 1 << 26
 BATCH_BYTES = 8 << 30            # of the batched fit's workspace (every head's key space at once)
@@ -95,43 +99,70 @@ BATCH_BYTES = 8 << 30            # of the batched fit's workspace (every head's 
 
 def _fit_batched(pk: torch.Tensor, *, seed: int, fit_n: int, c: int, iters: int, align: int, router_pass: bool):
     """The whole fit and layout of every KV head in one call, with one host read at the end
-    (sbsa_kmeans_fit).  Returns (sizes, indptr, posting rows, inverse, codebooks, width), or
-    None: a shape the call does not take, or a head that left clusters empty in more
-    iterations than restarts are drawn ahead for."""
+    (sbsa_kmeans_fit_counted).  A head that left clusters empty in more iterations than
+    restarts are drawn ahead for is fitted again alone, with a restart drawn for every
+    iteration, and so are the heads after it, until one needs no more: the rest follow
+    together.  (Keys with 90 distinct rows, where every iteration of every head leaves clusters
+    empty, 1 / 2 / 4 / 8 heads of D = 128 at 8192 positions: 767 / 1206 / 2326 / 5545 us, head
+    after head 1512 / 2886 / 5373 / 10668.)  Returns (sizes, indptr, posting rows, inverse,
+    codebooks, width), or None: a shape the call does not take, or more restarts than it draws."""
     length, hkv, dim = pk.shape
     dev = pk.device
     fits = hkv + RESTARTS_AHEAD * (hkv * (hkv - 1) // 2)
     if (not 0 <= seed or fits > BATCH_FITS or fits * fit_n * c > BATCH_WORK or dim not in (64, 128, 256)
             or pk.stride(0) % 8 or pk.stride(1) % 8 or pk.data_ptr() % 16 or length >= 1 << 27 or iters < 1):
         return None
-    shape = (length, fit_n, hkv, c, dim, RESTARTS_AHEAD, iters)
-    ws_bytes = _lib.query("sbsa_kmeans_fit_workspace_bytes", *shape)
+    ws_bytes = _lib.query("sbsa_kmeans_fit_workspace_bytes", length, fit_n, hkv, c, dim, RESTARTS_AHEAD, iters)
     if ws_bytes == 0 or ws_bytes > BATCH_BYTES:
         return None
-    n_draws = _lib.query("sbsa_kmeans_draw_ints", fit_n, hkv, c, RESTARTS_AHEAD)
-    # drawn into pinned memory, the draws' scratch behind them (memory the host allocator
-    # keeps: fresh pages would cost more than the draws)
-    n_scratch = _lib.query("sbsa_kmeans_draw_scratch_ints", length, fit_n, hkv, RESTARTS_AHEAD)
-    host = torch.empty(n_draws + n_scratch, dtype=torch.int32, pin_memory=True)
-    _lib.call("sbsa_kmeans_draws", seed & 0xffffffff, length, fit_n, hkv, c, RESTARTS_AHEAD, host.data_ptr(),
-              host[n_draws:].data_ptr())
-    draws = host[:n_draws].to(dev, non_blocking=True)
-    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
+
+    def drawn(first, restarts, heads, ahead):
+        """The draws of the heads from ``first`` on, after ``restarts`` restarts of those before them."""
+        n_draws = _lib.query("sbsa_kmeans_draw_ints", fit_n, heads, c, ahead)
+        # drawn into pinned memory, the draws' scratch behind them (memory the host allocator
+        # keeps: fresh pages would cost more than the draws)
+        n_scratch = _lib.query("sbsa_kmeans_draw_scratch_ints", length, fit_n, heads, ahead)
+        host = torch.empty(n_draws + n_scratch, dtype=torch.int32, pin_memory=True)
+        _lib.call("sbsa_kmeans_draws_after", seed & 0xffffffff, first, restarts, length, fit_n, heads, c, ahead,
+                  host.data_ptr(), host[n_draws:].data_ptr())
+        return host[:n_draws].to(dev, non_blocking=True)
+
+    first = restarts = width = 0
+    heads, ahead = hkv, RESTARTS_AHEAD
+    draws = drawn(first, restarts, heads, ahead)
     cap = length + c * (align - 1)
     posting = torch.empty(hkv, cap, dtype=torch.int32, device=dev)
     inverse = torch.empty(hkv, length, dtype=torch.int32, device=dev)
     sizes = torch.empty(hkv, c, dtype=torch.int32, device=dev)
     indptr = torch.empty(hkv, c + 1, dtype=torch.int32, device=dev)
-    totals = torch.empty(hkv + 1, dtype=torch.int32, device=dev)
     codebooks = torch.empty(hkv, 2, c, dim // 2, dtype=pk.dtype, device=dev)
-    _lib.call("sbsa_kmeans_fit", _lib.ptr(pk), length, pk.stride(0), pk.stride(1), hkv, dim, int(router_pass),
-              _lib.ptr(draws), fit_n, c, RESTARTS_AHEAD, iters, align, _lib.ptr(sizes), _lib.ptr(indptr),
-              _lib.ptr(posting), cap, _lib.ptr(inverse), _lib.ptr(totals), _lib.ptr(codebooks), _lib.ptr(ws),
-              ws_bytes, _lib.stream(dev))
-    *widths, valid_heads = totals.tolist()          # the one host read
-    if valid_heads < hkv:
-        return None
-    return sizes, indptr, posting, inverse, codebooks, max(widths)
+
+    def rest(t):
+        return _lib.ptr(t[first:] if first else t)
+
+    while True:
+        ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
+        totals = torch.empty(heads + 2, dtype=torch.int32, device=dev)
+        _lib.call("sbsa_kmeans_fit_counted", _lib.ptr(pk[:, first:] if first else pk), length, pk.stride(0),
+                  pk.stride(1), heads, dim, int(router_pass), _lib.ptr(draws), fit_n, c, ahead, iters, align,
+                  rest(sizes), rest(indptr), rest(posting), cap, rest(inverse), _lib.ptr(totals),
+                  _lib.ptr(totals[heads + 1:]), rest(codebooks), _lib.ptr(ws), ws_bytes, _lib.stream(dev))
+        *widths, valid, made = totals.tolist()          # the one host read
+        width = max([width, *widths[:valid]])
+        first += valid
+        restarts += made
+        if first == hkv:
+            return sizes, indptr, posting, inverse, codebooks, width
+        if valid == heads and made <= RESTARTS_AHEAD:
+            heads, ahead = hkv - first, RESTARTS_AHEAD
+        elif valid == 0 and heads == 1 and ahead == min(iters, RESTARTS_MOST):
+            return None                                 # more restarts than a call can draw
+        else:
+            # the next head alone, until one needs no more than are drawn ahead again
+            heads, ahead = 1, min(iters, RESTARTS_MOST)
+        draws = drawn(first, restarts, heads, ahead)
+        # (fewer heads: no more than before)
+        ws_bytes = _lib.query("sbsa_kmeans_fit_workspace_bytes", length, fit_n, heads, c, dim, ahead, iters)
 
 
 @dataclass
