@@ -19,14 +19,16 @@ def pytest_configure(config):
 
 
 @pytest.fixture
-def limit_memory():
-    """Leaves torch's GPU allocator ``extra`` bytes past what is in use (a limit of the allocator)."""
+def limit_memory(monkeypatch):
+    """Lets torch.empty refuse GPU memory past a size, as the allocator does where it is short."""
     import torch
+    real = torch.empty
 
-    def limit(extra):
-        torch.cuda.synchronize()
-        torch.cuda.empty_cache()
-        total = torch.cuda.get_device_properties(0).total_memory
-        torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + extra) / total)
-    yield limit
-    torch.cuda.set_per_process_memory_fraction(1.0)
+    def limit(most):
+        def empty(*size, **kw):
+            t = real(*size, **{**kw, "device": "meta", "pin_memory": False})
+            if torch.device(kw.get("device") or "cpu").type == "cuda" and t.numel() * t.element_size() > most:
+                raise torch.OutOfMemoryError("no room")
+            return real(*size, **kw)
+        monkeypatch.setattr(torch, "empty", empty)
+    return limit
