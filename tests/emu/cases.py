@@ -74,6 +74,38 @@ def dense_chunk(length: int, hq: int, hkv: int, d: int, cs: int, ce: int, seed: 
 
 
 
+def pair_chunk(d: int, g: int, qn: int, grid: int, seed: int) -> None:
+    """A sparse chunk through the two-block form of the attention (an explicit grid), its blocks
+    working through several items: runs around the 32-key tile, one KV head, some keys that
+    tower over their run's first tile (those items are run again)."""
+    from semblo_amd.kv_outer import kv_outer_attention
+    d, g, qn, grid, seed = map(int, (d, g, qn, grid, seed))
+    gen = torch.Generator().manual_seed(seed)
+    lens = torch.tensor([33, 0, 64, 1, 70] + [0] * 27)
+    indptr = torch.zeros(1, 33, dtype=torch.int64)
+    indptr[0, 1:] = ((lens + 15) // 16 * 16).cumsum(0)
+    packed = torch.randn(2, int(indptr[0, -1]), 1, d, generator=gen)
+    q = torch.randn(qn, g, d, generator=gen)
+    u = torch.randn(d, generator=gen)
+    q = q + 3 * u
+    packed[0, 40::41] = 3 * u
+    q, packed = q.to(torch.bfloat16), packed.to(torch.bfloat16)
+    kw, vw = (torch.randn(qn, 1, d, generator=gen).to(torch.bfloat16) for _ in range(2))
+    sel = torch.rand(qn, 1, 32, generator=gen) < 0.6
+    words = (sel.long() << torch.arange(32)).sum(-1, keepdim=True)
+    words = torch.where(words >= 2 ** 31, words - 2 ** 32, words).to(torch.int32)
+    out, stats = kv_outer_attention(q, packed, words, lens[None].int(), indptr.int(), sm_scale=d ** -0.5,
+                                    local_kv=(kw, vw), chunk_start=500, wstart=500, grid=grid)
+    assert stats["partials"] == int((sel & (lens > 0)).sum())
+    rows = torch.cat([torch.arange(int(indptr[0, i]), int(indptr[0, i] + lens[i])) for i in range(32)])
+    owner = torch.repeat_interleave(torch.arange(32), lens)
+    keys = torch.cat([sel[:, 0][:, owner], torch.ones(qn, qn, dtype=torch.bool).tril()], dim=1)
+    k, v = torch.cat([packed[0, rows], kw]), torch.cat([packed[1, rows], vw])
+    want = attention_reference(q, keys[:, None], k, v, d ** -0.5)
+    err = assert_close_bf16(out, want, f"emulated pair chunk D={d} G={g} Q={qn} grid={grid}")
+    print(f"pair chunk D={d} G={g} Q={qn} grid={grid}: max err {err:.3g}")
+
+
 def decode_steps(length: int, hq: int, hkv: int, d: int, seed: int, steps: int = 4,
                  splits: int = 8, target: int = 0) -> None:
     """Decode steps over the prompt's selection and the suffix store

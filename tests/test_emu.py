@@ -59,6 +59,11 @@ def test_emulated_dense_prefix_chunk():
     _run("dense_chunk", 256, 8, 2, 128, 128, 191, 3)
 
 
+def test_emulated_two_block_attention_over_several_items():
+    _run("pair_chunk", 256, 8, 40, 1, 3)
+    _run("pair_chunk", 128, 2, 200, 8, 4)       # a block's first two items are its own
+
+
 @long_case
 def test_emulated_sparse_chunk():
     _run("sparse_chunk", 1024, 8, 2, 128, 512, 767, 1, 2)

@@ -2,7 +2,9 @@
 whose lengths sit around multiples of the 32-key tile, work items with a full, a nearly
 empty and a single-query last tile of queries, for every head grouping and both head
 dimensions, on the whole grid and on one of 8 blocks (each block then works through
-many items).  Against fp64 attention over the explicit key sets."""
+many items, in the two-block form, which dense chunks of this size take only with an
+explicit grid; test_gpu_attend_forms.py has the launches that pick it by themselves).  Against
+fp64 attention over the explicit key sets."""
 from __future__ import annotations
 
 import pytest
@@ -59,7 +61,8 @@ def test_sparse_chunk_at_tile_edges(hkv, g, d, qn, grid):
                                            (0, 65, -1), (200, 129, -1)])
 @pytest.mark.parametrize("transposed,tower", [(False, False), (True, False), (False, True)])
 def test_dense_chunk_at_tile_edges(hkv, g, d, start, qn, grid, transposed, tower):
-    """Both kernel forms (grid -1 asks for the one that leaves room), also with the output's
+    """Both kernel forms (the two-block one at grid 8, the other at these sizes and where grid -1
+    asks for the one that leaves room), also with the output's
     heads outside its queries (a strided output) and with keys that tower over the first
     tile's (every 61st lies along the queries' common direction: the items are redone)."""
     from semblo_amd.kv_outer import dense_causal_attention
