@@ -203,7 +203,8 @@ int sbsa_causal_sizes(const int32_t* posting, int64_t width, const int32_t* indp
  * each (head, cluster) with nvis > 0, the ascending query ids whose qmask has
  * it.  rev_counts [Hkv*C], rev_indptr [Hkv*C + 1], nnz (device int64), qvals
  * [qvals_cap >= Q*Hkv*C], qrank [Q, Hkv, C] (rank of q in the cluster's list,
- * written where selected).  Deterministic, no atomics.  With qvals_cap at least
+ * written where selected).  Deterministic, no atomics; nnz may lie in pinned host
+ * memory (it is written once, by the scan).  With qvals_cap at least
  * sbsa_reverse_index_ints(Q, Hkv, C), the room past the lists holds counts of the
  * faster form. */
 int64_t sbsa_reverse_index_ints(int num_queries, int num_kv_heads, int num_clusters);

@@ -726,9 +726,10 @@ __global__ __launch_bounds__(256, 1) void attn_items_kernel(AttnArgs a) {
 // - nothing that only the boundary uses lives across the tile loop (the lane
 //   number is made opaque there): a spilled register's reload would wait for
 //   every load and store in flight.
-// Bound at D = 256 by LDS: 128 KB of operand reads and 32 KB of tile writes per
-// 128 x 32 tile, 1280 cycles at 128 B/clk against 1024 of matrix work (a dense
-// chunk takes about 1300).  One MI355X, same inputs, former form -> this one: a
+// Bound by the matrix cores at the clock that the chip holds under this load: by the
+// counters they are busy 78-79 % of the cycles of a dense chunk (D = 256, 1024 items),
+// the LDS index unit 39 %; 46-57 % in sparse chunks, whose items are 7-17 tiles long
+// (item ends, and the last items alone on their units).  One MI355X, same inputs, former form -> this one: a
 // dense chunk of 8192 queries at 24576, 3564 -> 2967 us (1080 -> 1297 TFLOP/s;
 // an 8192^3 bf16 matrix product reaches 1313 there); a sparse chunk of 8192 at
 // 114688 (980K entries), 2328 -> 1846 us (750 -> 946 TFLOP/s); D = 128, a sparse
