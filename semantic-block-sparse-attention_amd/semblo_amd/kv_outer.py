@@ -21,6 +21,7 @@ once everything is enqueued.
 """
 from __future__ import annotations
 
+import functools
 import os
 
 import torch
@@ -414,6 +415,7 @@ def _zero_counts(n: int, dev) -> torch.Tensor:
 DENSE_CLUSTERS = 32
 
 
+@functools.lru_cache(maxsize=64)
 def dense_launch_queries(num_kv_heads: int, q_per_kv: int) -> int:
     """The most queries ``dense_causal_attention`` takes in one call."""
     return _lib.query("sbsa_prefill_items_max_queries", num_kv_heads, DENSE_CLUSTERS, queries_per_item(q_per_kv))

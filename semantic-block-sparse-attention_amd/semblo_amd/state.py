@@ -125,11 +125,11 @@ def _fit_batched(pk: torch.Tensor, *, seed: int, fit_n: int, c: int, iters: int,
         host = torch.empty(n_draws + n_scratch, dtype=torch.int32, pin_memory=True)
         _lib.call("sbsa_kmeans_draws_after", seed & 0xffffffff, first, restarts, length, fit_n, heads, c, ahead,
                   host.data_ptr(), host[n_draws:].data_ptr())
-        return host[:n_draws].to(dev, non_blocking=True)
+        return host, host[:n_draws].to(dev, non_blocking=True)      # `host` is given back after the read
 
     first = restarts = width = 0
     heads, ahead = hkv, RESTARTS_AHEAD
-    draws = drawn(first, restarts, heads, ahead)
+    host, draws = drawn(first, restarts, heads, ahead)
     cap = length + c * (align - 1)
     posting = torch.empty(hkv, cap, dtype=torch.int32, device=dev)
     inverse = torch.empty(hkv, length, dtype=torch.int32, device=dev)
@@ -160,7 +160,7 @@ def _fit_batched(pk: torch.Tensor, *, seed: int, fit_n: int, c: int, iters: int,
         else:
             # the next head alone, until one needs no more than are drawn ahead again
             heads, ahead = 1, min(iters, RESTARTS_MOST)
-        draws = drawn(first, restarts, heads, ahead)
+        host, draws = drawn(first, restarts, heads, ahead)
         # (fewer heads: no more than before)
         ws_bytes = _lib.query("sbsa_kmeans_fit_workspace_bytes", length, fit_n, heads, c, dim, ahead, iters)
 
